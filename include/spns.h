@@ -219,7 +219,8 @@ int spns_device_memory(int32_t device, int64_t *free_bytes, int64_t *total_bytes
 int spns_last_step_ms(spns_ctx *ctx, double *ms);
 /* Runs nsteps steps launched pass by pass with HIP events between the passes
  * on the context's stream and returns the mean ms of each pass in ms[0..7]:
- * clear, inv_y, inv_x, z pass, fwd_x, fwd_y, epilogue, finalize.  The steps
+ * clear (nothing runs there: about 0), inv_y, inv_x, z pass, fwd_x, fwd_y,
+ * epilogue, finalize.  The steps
  * advance the solution like spns_step (no reference counterpart). */
 int spns_profile_passes(spns_ctx *ctx, int32_t nsteps, double *ms);
 

@@ -213,9 +213,8 @@ struct spns_ctx {
     double* hist_partial = nullptr;
     double* om_partial = nullptr;
     double* ed_partial = nullptr;  // [grid_epi] direct E sums of a reduce (QA energy check)
-    double* skew_partial = nullptr;
-    unsigned long long* mv = nullptr;  // [2]
-    unsigned long long* mv_save = nullptr;  // [2] (the QA energy check keeps the CFL maxima)
+    double* z_partial = nullptr;  // [grid_z][4] the z pass's block partials
+    int* ticket = nullptr;        // the finalize's arrival count
     // x1v (device int): X1 slots 0-5 hold u_c and d/dy u_c of the current
     // state, written by the previous step's k_yepi_inv; the step's inverse y
     // pass then does nothing.  yinv: the step runs k_yepi_inv (grid_yinv).
@@ -322,16 +321,15 @@ struct spns_ctx {
         alloc((void**)&hist_partial, sizeof(double) * (size_t)grid_epi * nbins);
         alloc((void**)&om_partial, sizeof(double) * grid_epi);
         alloc((void**)&ed_partial, sizeof(double) * grid_epi);
-        alloc((void**)&skew_partial, sizeof(double) * 2 * grid_z);
-        alloc((void**)&mv, sizeof(unsigned long long) * 2);
-        alloc((void**)&mv_save, sizeof(unsigned long long) * 2);
+        alloc((void**)&z_partial, sizeof(double) * 4 * grid_z);
+        alloc((void**)&ticket, sizeof(int));
         alloc((void**)&x1v, sizeof(int));
         alloc((void**)&ek, sizeof(double) * nbins);
         alloc((void**)&ft, sizeof(double) * (nbins + 1));
-        HIPCHK(hipMemsetAsync(skew_partial, 0, sizeof(double) * 2 * grid_z, st));
+        HIPCHK(hipMemsetAsync(z_partial, 0, sizeof(double) * 4 * grid_z, st));
         HIPCHK(hipMemsetAsync(X1, 0, (size_t)n_x1 * x1_slot * tsz, st));
         HIPCHK(hipMemsetAsync(X2, 0, (size_t)9 * x2_slot * tsz, st));
-        HIPCHK(hipMemsetAsync(mv, 0, sizeof(unsigned long long) * 2, st));
+        HIPCHK(hipMemsetAsync(ticket, 0, sizeof(int), st));
         HIPCHK(hipMemsetAsync(x1v, 0, sizeof(int), st));
         for (int c = 0; c < 3; c++) {
             HIPCHK(hipMemsetAsync(uk[c], 0, sb, st));
@@ -423,7 +421,7 @@ struct spns_ctx {
         if (graph) hipGraphExecDestroy(graph);
         for (int c = 0; c < 3; c++) { hipFree(uk[c]); hipFree(R[c]); hipFree(ukprev[c]); }
         hipFree(X1); hipFree(X2); hipFree(twx); hipFree(twy); hipFree(twz);
-        hipFree(scal); hipFree(hist_partial); hipFree(om_partial); hipFree(ed_partial); hipFree(skew_partial); hipFree(mv); hipFree(mv_save);
+        hipFree(scal); hipFree(hist_partial); hipFree(om_partial); hipFree(ed_partial); hipFree(z_partial); hipFree(ticket);
         hipFree(x1v);
         hipFree(ek); hipFree(forced); hipFree(ft); hipFree(invspec);
         if (ev0) hipEventDestroy(ev0);
@@ -509,9 +507,7 @@ struct spns_ctx {
         z.npencil = (int64_t)My * Mx;
         z.Ax = Ax; z.Ay = Ay; z.Az = Az;
         z.ct = ct;
-        z.maxvel_bits = mv;
-        z.maxvel_sa_bits = mv + 1;
-        z.skew_partial = skew_partial;
+        z.z_partial = z_partial;
         z.phys = phys;
         z.tw = twz;
         if (z.npencil * nk3p > x2_slot || nk3 > nk3p) throw Error(SPNS_EINVAL, "z pass exceeds its buffer");
@@ -664,8 +660,8 @@ struct spns_ctx {
         f.scal = scal;
         f.flags = flags;
         f.nbins = nbins; f.nblk_epi = grid_epi; f.nblk_z = grid_z;
-        f.hist_partial = hist_partial; f.om_partial = om_partial; f.ed_partial = ed_partial; f.skew_partial = skew_partial;
-        f.maxvel_bits = mv; f.maxvel_sa_bits = mv + 1;
+        f.hist_partial = hist_partial; f.om_partial = om_partial; f.ed_partial = ed_partial; f.z_partial = z_partial;
+        f.ticket = ticket;
         f.ek = ek;
         f.kfmin = cfg.force_kmin; f.kfmax = cfg.force_kmax; f.force_eps = cfg.force_on ? cfg.force_eps : 0.0;
         f.Ax = Ax; f.Ay = Ay; f.Az = Az; f.C_At = cfg.C_At; f.fixed_dt = cfg.fixed_dt;
@@ -683,7 +679,6 @@ struct spns_ctx {
 
     void enqueue_step()
     {
-        HIPCHK(launch_clear(mv, mv + 1, st));
         inv_y(false);
         inv_x(false);
         zpass(0, nullptr);
@@ -709,7 +704,6 @@ struct spns_ctx {
         const DevScalars before = read_scalars();
         std::vector<double> bins(nbins);
         HIPCHK(hipMemcpyAsync(bins.data(), ek, sizeof(double) * nbins, hipMemcpyDeviceToHost, st));
-        HIPCHK(hipMemcpyAsync(mv_save, mv, sizeof(unsigned long long) * 2, hipMemcpyDeviceToDevice, st));
         reduce_state();
         velocity_pass(nullptr);
         const DevScalars after = read_scalars();
@@ -718,15 +712,14 @@ struct spns_ctx {
         *ek_spns = after.ek;
         write_scalars(before);
         HIPCHK(hipMemcpyAsync(ek, bins.data(), sizeof(double) * nbins, hipMemcpyHostToDevice, st));
-        HIPCHK(hipMemcpyAsync(mv, mv_save, sizeof(unsigned long long) * 2, hipMemcpyDeviceToDevice, st));
         HIPCHK(hipStreamSynchronize(st));
     }
 
     // u,v,w from the state: CFL maxima (and the physical field if phys)
     // Physical velocity of the state at the start of the last step (the
-    // current state before any step) into phys.  The maxima the z pass
-    // accumulates stay in mv, which every step and velocity pass clears and
-    // only a finalize with FIN_MAXVEL reads, so the CFL state is unchanged.
+    // current state before any step) into phys.  The maxima the z pass leaves
+    // in z_partial are read only by a finalize with FIN_MAXVEL, which always
+    // follows a z pass of its own, so the CFL state is unchanged.
     void velocity_step_start(void* phys)
     {
         const DevScalars sc = read_scalars();
@@ -740,7 +733,6 @@ struct spns_ctx {
 
     void velocity_pass(void* phys)
     {
-        HIPCHK(launch_clear(mv, mv + 1, st));
         inv_y(true);
         inv_x(true);
         zpass(1, phys);
@@ -897,7 +889,6 @@ struct spns_batch {
         ZArgs z;
         EpiArgs epi;
         FinArgs fin;
-        ClearArgs clr;
     };
     SlotArgs* hs = nullptr;
     // pinned copies of each slot's device scalars, refreshed after every
@@ -909,7 +900,6 @@ struct spns_batch {
     ZArgs* d_z = nullptr;
     EpiArgs* d_epi = nullptr;
     FinArgs* d_fin = nullptr;
-    ClearArgs* d_clr = nullptr;
     int* d_left = nullptr;
     hipGraphExec_t graph = nullptr;
     std::string err;
@@ -936,7 +926,7 @@ struct spns_batch {
         al((void**)&d_invy2, sizeof(StridedArgs) * n);
         al((void**)&d_fwdx, sizeof(StridedArgs) * n); al((void**)&d_fwdy, sizeof(StridedArgs) * n);
         al((void**)&d_z, sizeof(ZArgs) * n); al((void**)&d_epi, sizeof(EpiArgs) * n);
-        al((void**)&d_fin, sizeof(FinArgs) * n); al((void**)&d_clr, sizeof(ClearArgs) * n);
+        al((void**)&d_fin, sizeof(FinArgs) * n);
         al((void**)&d_left, sizeof(int) * n);
         SlotSteps z{};
         HIPCHK(launch_set_left(d_left, z, nslots, st));
@@ -948,7 +938,7 @@ struct spns_batch {
         if (st) hipStreamSynchronize(st);
         if (graph) hipGraphExecDestroy(graph);
         hipFree(d_invy); hipFree(d_invx); hipFree(d_fwdx); hipFree(d_fwdy); hipFree(d_invy2); hipFree(d_z); hipFree(d_epi);
-        hipFree(d_fin); hipFree(d_clr); hipFree(d_left);
+        hipFree(d_fin); hipFree(d_left);
         if (hs) hipHostFree(hs);
         if (hsc) hipHostFree(hsc);
         if (ev) hipEventDestroy(ev);
@@ -998,12 +988,11 @@ struct spns_batch {
         a.epi = c->epi_args(EPI_STEP);
         a.fin = c->fin_args(FIN_REDUCE | FIN_SKEW | FIN_MAXVEL | FIN_DT | FIN_ADVANCE);
         a.fin.nblk_epi = c->yinv ? c->grid_yinv : c->grid_yepi > 0 ? c->grid_yepi : c->grid_epi;
-        a.clr = ClearArgs{c->mv, c->mv + 1};
         auto up = [&](void* d, const void* h, size_t bytes) { HIPCHK(hipMemcpyAsync(d, h, bytes, hipMemcpyHostToDevice, st)); };
         up(d_invy + s, &a.invy, sizeof(StridedArgs)); up(d_invx + s, &a.invx, sizeof(StridedArgs));
         up(d_z + s, &a.z, sizeof(ZArgs)); up(d_fwdx + s, &a.fwdx, sizeof(StridedArgs));
         up(d_fwdy + s, &a.fwdy, sizeof(StridedArgs)); up(d_epi + s, &a.epi, sizeof(EpiArgs));
-        up(d_fin + s, &a.fin, sizeof(FinArgs)); up(d_clr + s, &a.clr, sizeof(ClearArgs));
+        up(d_fin + s, &a.fin, sizeof(FinArgs));
         up(d_invy2 + s, &a.invy2, sizeof(StridedArgs));
         HIPCHK(hipMemcpyAsync(hsc + s, c->scal, sizeof(DevScalars), hipMemcpyDeviceToHost, st));
         HIPCHK(hipEventRecord(ev_sc, st));
@@ -1032,8 +1021,6 @@ struct spns_batch {
         const int p = c->prec;
         auto bl = [&](const void* a, const void* a2 = nullptr) { return BatchLaunch{a, a2, d_left, nslots}; };
         BatchLaunch b;
-        b = bl(d_clr);
-        HIPCHK(launch_clear(nullptr, nullptr, st, &b));
         b = bl(d_invy);
         HIPCHK(launch_strided(c->My, p, 1, p == PREC_FP64, +1, hs[slot_of(c)].invy, c->nk1, st, &b));
         b = bl(d_invx);
@@ -1732,7 +1719,6 @@ int spns_profile_passes(spns_ctx* ctx, int32_t nsteps, double* ms)
     try {
         for (int s = 0; s < nsteps; s++) {
             HIPCHK(hipEventRecord(ev[0], ctx->st));
-            HIPCHK(launch_clear(ctx->mv, ctx->mv + 1, ctx->st));
             HIPCHK(hipEventRecord(ev[1], ctx->st));
             ctx->inv_y(false);
             HIPCHK(hipEventRecord(ev[2], ctx->st));

@@ -57,9 +57,7 @@ struct ZArgs {
     int64_t npencil;
     double Ax, Ay, Az;  // CFL divisors (src/HIT_LES.h:56-58)
     double ct;          // (C_Smag*delta)^2 (src/HIT_LES.cpp:132)
-    unsigned long long* maxvel_bits;
-    unsigned long long* maxvel_sa_bits;
-    double* skew_partial;  // [gridDim.x][2]: MODE 0 sums of (du/dx)^2, (du/dx)^3; MODE 1 sum of u.u, 0
+    double* z_partial;  // [gridDim.x][4]: MODE 0 sums of (du/dx)^2, (du/dx)^3; MODE 1 sum of u.u, 0; then the CFL maxima
     void* phys;            // MODE 1: optional [3][npencil][L] physical export
     const void* tw;
 };
@@ -108,9 +106,8 @@ struct FinArgs {
     const double* hist_partial;
     const double* om_partial;
     const double* ed_partial;    // FIN_EFOUR: [nblk_epi] direct E partials
-    const double* skew_partial;  // [nblk_z][2]; after a velocity pass [b][0] holds sum u.u (FIN_EPHYS)
-    const unsigned long long* maxvel_bits;
-    const unsigned long long* maxvel_sa_bits;
+    const double* z_partial;  // [nblk_z][4]; after a velocity pass [b][0] holds sum u.u (FIN_EPHYS)
+    int* ticket;              // arrival count of the launch's blocks, 0 between launches
     double* ek;  // [nbins]
     int kfmin, kfmax;
     double force_eps;
@@ -142,11 +139,6 @@ struct RandArgs {
     int notcubic, Lx, Ly, Lz;
     uint64_t seed;
     double k0;
-};
-
-struct ClearArgs {
-    unsigned long long* a;
-    unsigned long long* b;
 };
 
 // A batched launch: one kernel over the slots of a shape class (runs with
@@ -196,7 +188,6 @@ hipError_t launch_set_int(int* p, int v, hipStream_t st);
 hipError_t launch_epilogue(int prec, const EpiArgs& a, int grid, hipStream_t st, const BatchLaunch* bl = nullptr);
 hipError_t launch_finalize(const FinArgs& a, hipStream_t st, const BatchLaunch* bl = nullptr);
 hipError_t launch_inv_spectra(int prec, const InvSpecArgs& a, int grid, double* out, hipStream_t st);
-hipError_t launch_clear(unsigned long long* a, unsigned long long* b, hipStream_t st, const BatchLaunch* bl = nullptr);
 hipError_t launch_set_left(int* left, const SlotSteps& s, int nslots, hipStream_t st);
 hipError_t launch_stream_copy(const void* in, void* out, int64_t bytes, int blocks, hipStream_t st);
 hipError_t launch_forcing(const double* ek, const double* forced, double* ft, int last_eff, const ShellArgs& a, hipStream_t st);

@@ -325,58 +325,68 @@ __global__ __launch_bounds__(NT) void k_sstage_b(const StridedArgs* __restrict__
 // ---------------------------------------------------------------------------
 // Block reductions
 // ---------------------------------------------------------------------------
-// Largest power of two <= n.
-__host__ __device__ constexpr int pow2_floor(int n)
+// Fixed-order sums and maxima: within a wave by shuffles (lane i with lane
+// i + 32, 16, ... 1), then over the waves in order through LDS.
+__device__ __forceinline__ double wave_sum(double v)
 {
-    int p = 1;
-    while (2 * p <= n) p *= 2;
-    return p;
+#pragma unroll
+    for (int s = 32; s > 0; s >>= 1) v = v + __shfl_down(v, s);
+    return v;
 }
 
-// Fixed-order block reductions for any NT: the NT - P top values (P the
-// largest power of two <= NT) are folded onto the first ones, then a tree.
+__device__ __forceinline__ double wave_max(double v)
+{
+#pragma unroll
+    for (int s = 32; s > 0; s >>= 1) v = fmax(v, __shfl_down(v, s));
+    return v;
+}
+
+// Sum over the block, in every thread; sh: NT / 64 doubles (free again on return).
 template <int NT>
 __device__ __forceinline__ double block_sum(double v, double* sh)
 {
-    constexpr int P = pow2_floor(NT);
-    const int t = threadIdx.x;
+    constexpr int NW = NT / 64;
+    v = wave_sum(v);
     __syncthreads();
-    sh[t] = v;
+    if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = v;
     __syncthreads();
-    if constexpr (P < NT) {
-        if (t < NT - P) sh[t] = sh[t] + sh[t + P];
-        __syncthreads();
-    }
-#pragma unroll
-    for (int s = P / 2; s > 0; s >>= 1) {
-        if (t < s) sh[t] = sh[t] + sh[t + s];
-        __syncthreads();
-    }
     double r = sh[0];
+    for (int w = 1; w < NW; w++) r = r + sh[w];
     __syncthreads();
     return r;
 }
 
+// The z pass's block partials, [4] per block: sums s2, s3; the block's CFL
+// velocity max(|u|/Ax, |v|/Ay, |w|/Az) (src/HIT_LES.cpp:393) and its sum form.
+// k_finalize takes the maxima over the blocks.  (A device-wide atomicMax per
+// block instead cost 50 of the 60 us of the 48^3 z pass: its 2304 blocks'
+// 64-bit atomics on one address are served one after the other.)  One LDS
+// exchange for all six values; sh: 6 NT / 64 doubles.
 template <int NT>
-__device__ __forceinline__ double block_max(double v, double* sh)
+__device__ __forceinline__ void z_partials(const ZArgs& a, double mu, double mv, double mw, double vsa, double s2, double s3, double* sh)
 {
-    constexpr int P = pow2_floor(NT);
-    const int t = threadIdx.x;
+    constexpr int NW = NT / 64;
+    const double r[6] = {wave_max(mu), wave_max(mv), wave_max(mw), wave_max(vsa), wave_sum(s2), wave_sum(s3)};
     __syncthreads();
-    sh[t] = v;
-    __syncthreads();
-    if constexpr (P < NT) {
-        if (t < NT - P) sh[t] = fmax(sh[t], sh[t + P]);
-        __syncthreads();
-    }
+    if ((threadIdx.x & 63) == 0) {
 #pragma unroll
-    for (int s = P / 2; s > 0; s >>= 1) {
-        if (t < s) sh[t] = fmax(sh[t], sh[t + s]);
-        __syncthreads();
+        for (int i = 0; i < 6; i++) sh[6 * (threadIdx.x >> 6) + i] = r[i];
     }
-    double r = sh[0];
     __syncthreads();
-    return r;
+    if (threadIdx.x == 0) {
+        double q[6];
+#pragma unroll
+        for (int i = 0; i < 6; i++) q[i] = sh[i];
+        for (int w = 1; w < NW; w++) {
+#pragma unroll
+            for (int i = 0; i < 6; i++) q[i] = i < 4 ? fmax(q[i], sh[6 * w + i]) : q[i] + sh[6 * w + i];
+        }
+        double* o = a.z_partial + 4 * (int64_t)blockIdx.x;
+        o[0] = q[4];
+        o[1] = q[5];
+        o[2] = fmax(q[0] / a.Ax, fmax(q[1] / a.Ay, q[2] / a.Az));
+        o[3] = q[3];
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -393,7 +403,7 @@ __global__ __launch_bounds__(NT) void k_zpass(ZArgs a)
 {
     constexpr int LD = 6;
     __shared__ cx<T> lds[L * LD];
-    __shared__ double red[NT];
+    __shared__ double red[6 * (NT / 64)];
     const cx<T>* tw = (const cx<T>*)a.tw;
     const int nk = a.nk3;
     const int t = threadIdx.x;
@@ -533,24 +543,7 @@ __global__ __launch_bounds__(NT) void k_zpass(ZArgs a)
         }
         __syncthreads();
     }
-    // -------- block reductions -> partials / atomics
-    const double bu = block_max<NT>((double)mu, red);
-    const double bv = block_max<NT>((double)mv, red);
-    const double bw = block_max<NT>((double)mw, red);
-    const double vmax = fmax(bu / iAx, fmax(bv / iAy, bw / iAz));  // src/HIT_LES.cpp:393
-    if (sa) vmax_sa = block_max<NT>(vmax_sa, red);
-    if (MODE <= 1) {
-        s2 = block_sum<NT>(s2, red);
-        s3 = block_sum<NT>(s3, red);
-    }
-    if (t == 0) {
-        atomicMax(a.maxvel_bits, (unsigned long long)__double_as_longlong(vmax));
-        atomicMax(a.maxvel_sa_bits, (unsigned long long)__double_as_longlong(vmax_sa));
-        if (MODE <= 1) {
-            a.skew_partial[2 * blockIdx.x] = s2;
-            a.skew_partial[2 * blockIdx.x + 1] = s3;
-        }
-    }
+    z_partials<NT>(a, (double)mu, (double)mv, (double)mw, vmax_sa, s2, s3, red);
 }
 
 
@@ -658,7 +651,7 @@ template <typename T, int L, int NT, int MODE, int LD = zstage_ld<MODE>()>
 __host__ __device__ constexpr size_t zstage_lds_bytes()
 {
     return sizeof(cx<T>) * ((size_t)L * LD + (size_t)(MODE == 1 ? 3 : 9) * zstage_spc<L>() + L) +
-           sizeof(double) * NT + 2 * 9 * sizeof(void*);
+           sizeof(double) * 6 * (NT / 64) + 2 * 9 * sizeof(void*);
 }
 
 template <typename T, int L, int NT, int MODE, int LD = zstage_ld<MODE>()>
@@ -688,7 +681,7 @@ __device__ __forceinline__ void zstage_body(const ZArgs& a)
     __shared__ __align__(16) cx<T> fbuf[L * LD];
     __shared__ __align__(16) cx<T> stg[NSRC * SPC];
     __shared__ __align__(16) cx<T> twl[L];
-    __shared__ double red[NT];
+    __shared__ double red[6 * (NT / 64)];
     __shared__ const cx<T>* srcp[9];
     __shared__ cx<T>* dstp[9];
     const int t = threadIdx.x;
@@ -859,23 +852,7 @@ __device__ __forceinline__ void zstage_body(const ZArgs& a)
         lds_barrier();  // every wave's copies are in; fbuf is free again
     }
     if constexpr (MODE == 2) return;  // a diagnostic pass: no CFL or skewness partials
-    const double bu = block_max<NT>((double)mu, red);
-    const double bv = block_max<NT>((double)mv, red);
-    const double bw = block_max<NT>((double)mw, red);
-    const double vmax = fmax(bu / iAx, fmax(bv / iAy, bw / iAz));  // src/HIT_LES.cpp:393
-    if (sa) vmax_sa = block_max<NT>(vmax_sa, red);
-    if (MODE <= 1) {
-        s2 = block_sum<NT>(s2, red);
-        s3 = block_sum<NT>(s3, red);
-    }
-    if (t == 0) {
-        atomicMax(a.maxvel_bits, (unsigned long long)__double_as_longlong(vmax));
-        atomicMax(a.maxvel_sa_bits, (unsigned long long)__double_as_longlong(vmax_sa));
-        if (MODE <= 1) {
-            a.skew_partial[2 * blockIdx.x] = s2;
-            a.skew_partial[2 * blockIdx.x + 1] = s3;
-        }
-    }
+    z_partials<NT>(a, (double)mu, (double)mv, (double)mw, vmax_sa, s2, s3, red);
 }
 
 template <typename T, int L, int NT, int MODE, int LD = zstage_ld<MODE>(), int MINW = 1, bool ZOPAQUE = (sizeof(T) == 4),
@@ -939,7 +916,7 @@ __device__ __forceinline__ void zfuse_body(const ZArgs& a)
     constexpr int NW = NT / 64;
     constexpr int EPS = 16 / (int)sizeof(cx<T>);
     constexpr int TWN = fft_twiddle_span<L, TWM>();
-    static_assert(L * LD * sizeof(cx<T>) >= NT * sizeof(double), "reduction scratch aliases the pair buffer");
+    static_assert(L * LD * sizeof(cx<T>) >= 6 * (NT / 64) * sizeof(double), "reduction scratch aliases the pair buffer");
     __shared__ __align__(16) cx<T> fbuf[L * LD];
     __shared__ __align__(16) cx<T> stg[9 * SPC];
     __shared__ __align__(16) cx<T> twl[TWN];
@@ -1136,20 +1113,7 @@ __device__ __forceinline__ void zfuse_body(const ZArgs& a)
         }
         prev = have ? pen : -1;
     }
-    double* red = (double*)fbuf;
-    const double bu = block_max<NT>((double)mu, red);
-    const double bv = block_max<NT>((double)mv, red);
-    const double bw = block_max<NT>((double)mw, red);
-    const double vmax = fmax(bu / iAx, fmax(bv / iAy, bw / iAz));  // src/HIT_LES.cpp:393
-    if (sa) vmax_sa = block_max<NT>(vmax_sa, red);
-    s2 = block_sum<NT>(s2, red);
-    s3 = block_sum<NT>(s3, red);
-    if (t == 0) {
-        atomicMax(a.maxvel_bits, (unsigned long long)__double_as_longlong(vmax));
-        atomicMax(a.maxvel_sa_bits, (unsigned long long)__double_as_longlong(vmax_sa));
-        a.skew_partial[2 * blockIdx.x] = s2;
-        a.skew_partial[2 * blockIdx.x + 1] = s3;
-    }
+    z_partials<NT>(a, (double)mu, (double)mv, (double)mw, vmax_sa, s2, s3, (double*)fbuf);
 }
 
 template <typename T, int L, int NT, int NKC = 0, int TWM = (sizeof(T) == 8 ? 1 : 2), bool ZOPAQUE = (sizeof(T) == 4)>
@@ -1231,7 +1195,7 @@ __global__ __launch_bounds__(256) void k_zwave(ZArgs a)
 {
     constexpr int E = L / 64, WPB = 4;
     __shared__ cx<T> ldsw[WPB][L];
-    __shared__ double red[256];
+    __shared__ double red[6 * 4];
     const int w = threadIdx.x >> 6, t = threadIdx.x & 63;
     cx<T>* lds = ldsw[w];
     const cx<T>* tw = (const cx<T>*)a.tw;
@@ -1314,21 +1278,7 @@ __global__ __launch_bounds__(256) void k_zwave(ZArgs a)
             wave_fwd_pair<T, L>(lds, tw, CZ, (const T*)nullptr, (cx<T>*)a.f[2], (cx<T>*)nullptr, off, nk);
         }
     }
-    const double bu = block_max<256>((double)mu, red);
-    const double bv = block_max<256>((double)mv, red);
-    const double bw = block_max<256>((double)mw, red);
-    const double vmax = fmax(bu / iAx, fmax(bv / iAy, bw / iAz));  // src/HIT_LES.cpp:393
-    if (sa) vmax_sa = block_max<256>(vmax_sa, red);
-    s2 = block_sum<256>(s2, red);
-    s3 = block_sum<256>(s3, red);
-    if (threadIdx.x == 0) {
-        atomicMax(a.maxvel_bits, (unsigned long long)__double_as_longlong(vmax));
-        atomicMax(a.maxvel_sa_bits, (unsigned long long)__double_as_longlong(vmax_sa));
-        {
-            a.skew_partial[2 * blockIdx.x] = s2;
-            a.skew_partial[2 * blockIdx.x + 1] = s3;
-        }
-    }
+    z_partials<256>(a, (double)mu, (double)mv, (double)mw, vmax_sa, s2, s3, red);
 }
 
 // ---------------------------------------------------------------------------
@@ -1552,7 +1502,7 @@ __device__ __forceinline__ void epilogue_body(const EpiArgs& a)
 {
     constexpr int NW = NT / 64;
     extern __shared__ double hist[];  // NW * nbins
-    __shared__ double red[NT];
+    __shared__ double red[NW];
     const int nb = a.nbins;
     for (int i = threadIdx.x; i < NW * nb; i += NT) hist[i] = 0.0;
     __syncthreads();
@@ -1669,7 +1619,7 @@ __device__ __forceinline__ void yepi_body(const StridedArgs& a, const EpiArgs& e
     constexpr int NOUTMAX = 2 * (L / 3) + 1;  // the launcher checks nout against it
     constexpr int Q = (NOUTMAX * TB + NT - 1) / NT;
     constexpr int STGN = yepi_stg_elems<T, L, TB, INV>();
-    static_assert(L * TB * sizeof(cx<T>) >= NT * sizeof(double), "reduction scratch aliases fbuf");
+    static_assert(L * TB * sizeof(cx<T>) >= (NT / 64) * sizeof(double), "reduction scratch aliases fbuf");
     __shared__ __align__(16) cx<T> fbuf[L * TB];
     __shared__ __align__(16) cx<T> stg[STGN];
     __shared__ __align__(16) cx<T> twl[TWN];
@@ -1866,65 +1816,82 @@ static __device__ double FuG(double x, double a, double b, double c, double x0, 
 
 // ---------------------------------------------------------------------------
 // Finalize: fixed-order sums of the partials; time step (src/HIT_LES.cpp:365-403)
+// With FIN_REDUCE the grid has one block per 64 shells: block x sums its
+// shells' block partials (wave w takes rows w, w + 16, ...), and the block that
+// arrives last does the rest.  What bounds it is the latency of dependent reads
+// of partials that other XCDs wrote, so rows are read eight at a time.  One
+// block over all shells took 60 us at 512^3 DNS (256 x 445 partials) and 51 at
+// 256^3 LES (1024 x 223); this 20 and 26.
+// Returns whether this block was the last one of its context's launch.
 // ---------------------------------------------------------------------------
 template <int NT>
-__device__ __forceinline__ void finalize_body(const FinArgs& a)
+__device__ __forceinline__ bool finalize_body(const FinArgs& a)
 {
-    __shared__ double red[NT];
+    constexpr int NW = NT / 64;
+    __shared__ double red[NW];
     DevScalars* s = a.scal;
     const int t = threadIdx.x;
     if (a.flags & FIN_REDUCE) {
-        // E(K): bins are split over NT/QB thread groups; each thread sums a
-        // fixed quarter of the block partials with 4 independent
-        // accumulators, and the quarters are combined in a fixed order.
-        constexpr int QB = 4;
-        __shared__ double q[QB][NT / QB];
-        const int lane = t % (NT / QB), quarter = t / (NT / QB);
-        const int per = (a.nblk_epi + QB - 1) / QB;
-        const int b0 = quarter * per, b1 = min(a.nblk_epi, b0 + per);
-        for (int K0 = 0; K0 < a.nbins; K0 += NT / QB) {
-            const int K = K0 + lane;
-            double acc[4] = {0.0, 0.0, 0.0, 0.0};
-            if (K < a.nbins) {
-                int b = b0;
-                for (; b + 3 < b1; b += 4) {
+        __shared__ double q[NW][64];
+        __shared__ int last;
+        const int lane = t & 63, w = t >> 6;
+        const int K = blockIdx.x * 64 + lane;
+        constexpr int U = 8;
+        double acc[U] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+        if (K < a.nbins) {
+            int b = w;
+            for (; b + (U - 1) * NW < a.nblk_epi; b += U * NW) {
 #pragma unroll
-                    for (int u = 0; u < 4; u++) acc[u] += a.hist_partial[(int64_t)(b + u) * a.nbins + K];
-                }
-                for (; b < b1; b++) acc[0] += a.hist_partial[(int64_t)b * a.nbins + K];
+                for (int u = 0; u < U; u++) acc[u] += a.hist_partial[(int64_t)(b + u * NW) * a.nbins + K];
             }
-            q[quarter][lane] = (acc[0] + acc[1]) + (acc[2] + acc[3]);
+            for (; b < a.nblk_epi; b += NW) acc[0] += a.hist_partial[(int64_t)b * a.nbins + K];
+        }
+        q[w][lane] = ((acc[0] + acc[1]) + (acc[2] + acc[3])) + ((acc[4] + acc[5]) + (acc[6] + acc[7]));
+        __syncthreads();
+        if (w == 0 && K < a.nbins) {
+            double e = q[0][lane];
+            for (int i = 1; i < NW; i++) e += q[i][lane];
+            a.ek[K] = e;
+        }
+        if (gridDim.x > 1) {
+            // publish this block's shells, then count it in; the last block
+            // sees every shell and leaves the counter at 0 for the next launch
+            __threadfence();
             __syncthreads();
-            if (quarter == 0 && K < a.nbins) a.ek[K] = ((q[0][lane] + q[1][lane]) + q[2][lane]) + q[3][lane];
+            if (t == 0) {
+                last = atomicAdd(a.ticket, 1) == (int)gridDim.x - 1;
+                if (last) atomicExch(a.ticket, 0);
+            }
+            __syncthreads();
+            if (!last) return false;
+            __threadfence();
+        } else {
             __syncthreads();
         }
-        double om = 0.0;
+        double om = 0.0, e = 0.0, ef = 0.0;
         for (int b = t; b < a.nblk_epi; b += NT) om += a.om_partial[b];
+        for (int k = t; k < a.nbins; k += NT) {
+            const double v = a.ek[k];
+            e += v;
+            if (k >= a.kfmin && k <= a.kfmax) ef += v;
+        }
         om = block_sum<NT>(om, red);
-        __syncthreads();
+        e = block_sum<NT>(e, red);
+        ef = block_sum<NT>(ef, red);
         if (t == 0) {
-            double e = 0.0;
-            for (int K = 0; K < a.nbins; K++) e += a.ek[K];
             s->ek = e;
             s->om = om;
             s->relambda = e / s->nu * sqrt(20.0 / 3.0 / om);
             // constant-power coefficient for the next step (src/HIT_LES.cpp:251-256)
-            double ef = 0.0;
-            for (int K = a.kfmin; K <= a.kfmax && K < a.nbins; K++) ef += a.ek[K];
             s->alpha = (ef > 1e-30) ? a.force_eps / (2.0 * ef) : 0.0;
         }
     }
     if (a.flags & FIN_SKEW) {
-        double s2[4] = {0.0, 0.0, 0.0, 0.0}, s3[4] = {0.0, 0.0, 0.0, 0.0};
-        int b = t;
-        for (; b + 3 * NT < a.nblk_z; b += 4 * NT) {
-#pragma unroll
-            for (int u = 0; u < 4; u++) { s2[u] += a.skew_partial[2 * (b + u * NT)]; s3[u] += a.skew_partial[2 * (b + u * NT) + 1]; }
-        }
-        for (; b < a.nblk_z; b += NT) { s2[0] += a.skew_partial[2 * b]; s3[0] += a.skew_partial[2 * b + 1]; }
-        double S2 = block_sum<NT>((s2[0] + s2[1]) + (s2[2] + s2[3]), red);
-        double S3 = block_sum<NT>((s3[0] + s3[1]) + (s3[2] + s3[3]), red);
-        if (t == 0) { s->skew2 = S2; s->skew3 = S3; }
+        double s2 = 0.0, s3 = 0.0;
+        for (int b = t; b < a.nblk_z; b += NT) { s2 += a.z_partial[4 * b]; s3 += a.z_partial[4 * b + 1]; }
+        s2 = block_sum<NT>(s2, red);
+        s3 = block_sum<NT>(s3, red);
+        if (t == 0) { s->skew2 = s2; s->skew3 = s3; }
     }
     if (a.flags & FIN_EFOUR) {
         double e = 0.0;
@@ -1934,15 +1901,25 @@ __device__ __forceinline__ void finalize_body(const FinArgs& a)
     }
     if (a.flags & FIN_EPHYS) {
         double e = 0.0;
-        for (int b = t; b < a.nblk_z; b += NT) e += a.skew_partial[2 * b];
+        for (int b = t; b < a.nblk_z; b += NT) e += a.z_partial[4 * b];
         e = block_sum<NT>(e, red);
         if (t == 0) s->ek_phys = e;
     }
-    if (t == 0) {
-        if (a.flags & FIN_MAXVEL) {
-            s->maxvel = __longlong_as_double((long long)*a.maxvel_bits);
-            s->maxvel_sa = __longlong_as_double((long long)*a.maxvel_sa_bits);
+    if (a.flags & FIN_MAXVEL) {
+        double v = 0.0, vs = 0.0;
+        for (int b = t; b < a.nblk_z; b += NT) { v = fmax(v, a.z_partial[4 * b + 2]); vs = fmax(vs, a.z_partial[4 * b + 3]); }
+        v = wave_max(v);
+        vs = wave_max(vs);
+        __shared__ double mx[NW][2];
+        if ((t & 63) == 0) { mx[t >> 6][0] = v; mx[t >> 6][1] = vs; }
+        __syncthreads();
+        if (t == 0) {
+            for (int w = 1; w < NW; w++) { v = fmax(v, mx[w][0]); vs = fmax(vs, mx[w][1]); }
+            s->maxvel = v;
+            s->maxvel_sa = vs;
         }
+    }
+    if (t == 0) {
         if (a.flags & FIN_DT) {
             const double nu = s->nu;
             if (a.sa) {
@@ -1973,6 +1950,7 @@ __device__ __forceinline__ void finalize_body(const FinArgs& a)
             s->iter = s->iter + 1;
         }
     }
+    return true;
 }
 
 template <int NT>
@@ -1982,25 +1960,15 @@ __global__ __launch_bounds__(NT) void k_finalize(FinArgs a)
 }
 
 // Batched form: the slot's step ends here, so its steps-left counter drops
-// by one (after every wave of the block has read it at entry).
+// by one: by the slot's last block, after every wave of its blocks has read it
+// at entry.
 template <int NT>
 __global__ __launch_bounds__(NT) void k_finalize_b(const FinArgs* __restrict__ arr, int* __restrict__ left)
 {
     if (left[blockIdx.y] <= 0) return;
-    finalize_body<NT>(arr[blockIdx.y]);
+    const bool last = finalize_body<NT>(arr[blockIdx.y]);
     __syncthreads();
-    if (threadIdx.x == 0) left[blockIdx.y] -= 1;
-}
-
-static __global__ void k_clear(unsigned long long* a, unsigned long long* b)
-{
-    if (threadIdx.x == 0) { *a = 0ull; *b = 0ull; }
-}
-
-static __global__ void k_clear_b(const ClearArgs* __restrict__ arr, const int* __restrict__ left)
-{
-    if (left[blockIdx.y] <= 0) return;
-    if (threadIdx.x == 0) { *arr[blockIdx.y].a = 0ull; *arr[blockIdx.y].b = 0ull; }
+    if (last && threadIdx.x == 0) left[blockIdx.y] -= 1;
 }
 
 // Streaming copy (the measured practical HBM ceiling beside the data-sheet
@@ -2789,21 +2757,12 @@ hipError_t launch_epilogue(int prec, const EpiArgs& a, int grid, hipStream_t st,
 
 hipError_t launch_finalize(const FinArgs& a, hipStream_t st, const BatchLaunch* bl)
 {
+    const unsigned g = (a.flags & FIN_REDUCE) ? (unsigned)((a.nbins + 63) / 64) : 1u;
     if (bl) {
-        hipLaunchKernelGGL((k_finalize_b<1024>), dim3(1, bl->nslots), dim3(1024), 0, st, (const FinArgs*)bl->args, bl->left);
+        hipLaunchKernelGGL((k_finalize_b<1024>), dim3(g, bl->nslots), dim3(1024), 0, st, (const FinArgs*)bl->args, bl->left);
         return hipGetLastError();
     }
-    hipLaunchKernelGGL((k_finalize<1024>), dim3(1), dim3(1024), 0, st, a);
-    return hipGetLastError();
-}
-
-hipError_t launch_clear(unsigned long long* a, unsigned long long* b, hipStream_t st, const BatchLaunch* bl)
-{
-    if (bl) {
-        hipLaunchKernelGGL(k_clear_b, dim3(1, bl->nslots), dim3(64), 0, st, (const ClearArgs*)bl->args, bl->left);
-        return hipGetLastError();
-    }
-    hipLaunchKernelGGL(k_clear, dim3(1), dim3(64), 0, st, a, b);
+    hipLaunchKernelGGL((k_finalize<1024>), dim3(g), dim3(1024), 0, st, a);
     return hipGetLastError();
 }
 
