@@ -11,6 +11,8 @@
 #include <mutex>
 #include <stdexcept>
 #include <string>
+#include <system_error>
+#include <thread>
 #include <vector>
 
 #include "../../include/spns.h"
@@ -94,6 +96,109 @@ void check_strided(StridedArgs& a, int A, const int64_t* in_cap, const int64_t* 
     }
 }
 
+}  // namespace
+
+// ===========================================================================
+// Copies between device memory and pageable host memory.  A large one goes
+// through pinned chunks that kThreads host threads fill or empty: the link moves
+// 57 GB/s, but one hipMemcpy into freshly allocated pages 10.3 (512 MiB), where
+// the page faults and the host's own copy are serial; this moves 32 (52 and
+// 170 MB; six or eight threads the same).  Small ones are one hipMemcpy: below
+// kSmall the threads cost more than they save.
+// The pinned memory (16 MiB) belongs to the owner and goes with it.
+// ===========================================================================
+namespace {
+struct HostCopy {
+    static constexpr int kThreads = 4;
+    static constexpr size_t kChunk = 2u << 20, kSmall = 8u << 20;
+    char* pin = nullptr;  // [kThreads][2][kChunk]
+    hipEvent_t ev[kThreads][2] = {};
+
+    // Complete on return.  Work queued on st before the call is finished first.
+    void copy(void* host, void* devp, size_t bytes, bool to_host, int device, hipStream_t st)
+    {
+        const hipMemcpyKind kind = to_host ? hipMemcpyDeviceToHost : hipMemcpyHostToDevice;
+        if (bytes < kSmall || !ready()) {
+            if (to_host) HIPCHK(hipMemcpyAsync(host, devp, bytes, kind, st));
+            else HIPCHK(hipMemcpyAsync(devp, host, bytes, kind, st));
+            HIPCHK(hipStreamSynchronize(st));
+            return;
+        }
+        const size_t nchunk = (bytes + kChunk - 1) / kChunk;
+        hipError_t err[kThreads] = {};
+        auto work = [&](int w) {
+            hipError_t e = hipSetDevice(device);
+            size_t pend[2] = {nchunk, nchunk};  // chunk whose copy uses each buffer
+            auto size = [&](size_t c) { return std::min(kChunk, bytes - c * kChunk); };
+            auto drain = [&](int b) {
+                if (pend[b] == nchunk) return;
+                if (e == hipSuccess) e = hipEventSynchronize(ev[w][b]);
+                if (e == hipSuccess && to_host) std::memcpy((char*)host + pend[b] * kChunk, buf(w, b), size(pend[b]));
+                pend[b] = nchunk;
+            };
+            int b = 0;
+            for (size_t c = w; c < nchunk && e == hipSuccess; c += kThreads, b ^= 1) {
+                drain(b);
+                if (e != hipSuccess) break;
+                char* d = (char*)devp + c * kChunk;
+                if (!to_host) std::memcpy(buf(w, b), (const char*)host + c * kChunk, size(c));
+                e = to_host ? hipMemcpyAsync(buf(w, b), d, size(c), kind, st) : hipMemcpyAsync(d, buf(w, b), size(c), kind, st);
+                if (e == hipSuccess) e = hipEventRecord(ev[w][b], st);
+                if (e == hipSuccess) pend[b] = c;
+            }
+            drain(b);
+            drain(b ^ 1);
+            err[w] = e;
+        };
+        std::thread th[kThreads];
+        for (int w = 1; w < kThreads; w++) {
+            try {
+                th[w] = std::thread(work, w);
+            } catch (const std::system_error&) {
+            }  // no thread to be had: its share is done below
+        }
+        work(0);
+        for (int w = 1; w < kThreads; w++) {
+            if (th[w].joinable()) th[w].join();
+            else work(w);
+        }
+        const hipError_t es = hipStreamSynchronize(st);
+        for (hipError_t e : err) HIPCHK(e);
+        HIPCHK(es);
+    }
+
+    bool ready()
+    {
+        if (pin) return true;
+        if (hipHostMalloc((void**)&pin, kThreads * 2 * kChunk, hipHostMallocDefault) != hipSuccess) {
+            (void)hipGetLastError();
+            pin = nullptr;
+            return false;
+        }
+        for (auto& e : ev)
+            for (hipEvent_t& q : e)
+                if (hipEventCreateWithFlags(&q, hipEventDisableTiming) != hipSuccess) {
+                    (void)hipGetLastError();
+                    q = nullptr;
+                    release();
+                    return false;
+                }
+        return true;
+    }
+
+    char* buf(int w, int b) const { return pin + ((size_t)w * 2 + b) * kChunk; }
+
+    void release()
+    {
+        for (auto& e : ev)
+            for (hipEvent_t& q : e) {
+                if (q) hipEventDestroy(q);
+                q = nullptr;
+            }
+        if (pin) hipHostFree(pin);
+        pin = nullptr;
+    }
+};
 }  // namespace
 
 // ===========================================================================
@@ -229,6 +334,7 @@ struct spns_ctx {
     int zkernel = ZK_STAGED;  // z-pass kernel (environment SPNS_ZPASS=staged|nofuse|block|wave overrides)
     hipGraphExec_t graph = nullptr;
     bool graph_ready = false;
+    HostCopy hcopy;
     std::string err;
     double last_ms = 0.0;
 
@@ -418,6 +524,7 @@ struct spns_ctx {
 
     void release()
     {
+        hcopy.release();
         if (graph) hipGraphExecDestroy(graph);
         for (int c = 0; c < 3; c++) { hipFree(uk[c]); hipFree(R[c]); hipFree(ukprev[c]); }
         hipFree(X1); hipFree(X2); hipFree(twx); hipFree(twy); hipFree(twz);
@@ -495,7 +602,7 @@ struct spns_ctx {
         HIPCHK(launch_strided(Mx, prec, prec == PREC_FP64, prec == PREC_FP64, +1, a, a.A, st));
     }
 
-    ZArgs zpass_args(void* phys)
+    ZArgs zpass_args(double* const* phys = nullptr)
     {
         ZArgs z{};
         for (int f = 0; f < 9; f++) z.f[f] = X2f(f);
@@ -508,12 +615,13 @@ struct spns_ctx {
         z.Ax = Ax; z.Ay = Ay; z.Az = Az;
         z.ct = ct;
         z.z_partial = z_partial;
-        z.phys = phys;
+        for (int c = 0; c < 3; c++) z.phys[c] = phys ? phys[c] : nullptr;
+        z.Mx = Mx; z.My = My;
         z.tw = twz;
         if (z.npencil * nk3p > x2_slot || nk3 > nk3p) throw Error(SPNS_EINVAL, "z pass exceeds its buffer");
         return z;
     }
-    void zpass(int mode, void* phys)
+    void zpass(int mode, double* const* phys = nullptr)
     {
         ZArgs z = zpass_args(phys);
         if (mode == 2) {
@@ -550,7 +658,7 @@ struct spns_ctx {
         cx<double>* const* src = (sc.iter > 0) ? ukprev : uk;
         inv_y(false, src);
         inv_x(false);
-        zpass(2, nullptr);
+        zpass(2);
         fwd_x(5);
         fwd_y(5);
         InvSpecArgs a{};
@@ -681,7 +789,7 @@ struct spns_ctx {
     {
         inv_y(false);
         inv_x(false);
-        zpass(0, nullptr);
+        zpass(0);
         fwd_x();
         FinArgs f = fin_args(FIN_REDUCE | FIN_SKEW | FIN_MAXVEL | FIN_DT | FIN_ADVANCE);
         f.nblk_epi = fwd_y_epilogue();
@@ -705,7 +813,7 @@ struct spns_ctx {
         std::vector<double> bins(nbins);
         HIPCHK(hipMemcpyAsync(bins.data(), ek, sizeof(double) * nbins, hipMemcpyDeviceToHost, st));
         reduce_state();
-        velocity_pass(nullptr);
+        velocity_pass();
         const DevScalars after = read_scalars();
         *ek_real = 0.5 * after.ek_phys / nf;  // src/HIT_LES.cpp:1236-1240
         *ek_four = after.ek_four;
@@ -720,7 +828,7 @@ struct spns_ctx {
     // current state before any step) into phys.  The maxima the z pass leaves
     // in z_partial are read only by a finalize with FIN_MAXVEL, which always
     // follows a z pass of its own, so the CFL state is unchanged.
-    void velocity_step_start(void* phys)
+    void velocity_step_start(double* const* phys)
     {
         const DevScalars sc = read_scalars();
         if (sc.iter > 0 && !keep_prev)
@@ -731,7 +839,7 @@ struct spns_ctx {
         zpass(1, phys);
     }
 
-    void velocity_pass(void* phys)
+    void velocity_pass(double* const* phys = nullptr)
     {
         inv_y(true);
         inv_x(true);
@@ -779,23 +887,29 @@ struct spns_ctx {
         HIPCHK(hipStreamSynchronize(st));
     }
 
-    void upload_state(const std::vector<std::complex<double>>& h)
+    // Compact rows [row0, row0 + nrow) of three pitched fields, packed in X2's
+    // space (free between passes; it holds all of them: retained modes fit the grid)
+    PackArgs pack_args(void* const* f, int64_t row0, int64_t nrow)
     {
-        // h: [3][nmodes]; modes masked by the length factors are zeroed
-        std::vector<std::complex<double>> m(h);
-        if (cfg.isNotCubic) {
-            for (int64_t q = 0; q < nmodes; q++) {
-                int i3 = (int)(q % nk3);
-                int64_t r = q / nk3;
-                int i1 = (int)(r % nk1), i2 = (int)(r / nk1);
-                int k1 = i1 <= nk1 / 2 ? i1 : i1 - nk1, k2 = i2 <= nk2 / 2 ? i2 : i2 - nk2, k3 = i3;
-                if ((k1 % cfg.Lx) || (k2 % cfg.Ly) || (k3 % cfg.Lz))
-                    for (int c = 0; c < 3; c++) m[c * nmodes + q] = 0.0;
-            }
-        }
-        for (int c = 0; c < 3; c++)
-            HIPCHK(hipMemcpy2DAsync(uk[c], sizeof(cx<double>) * nk3p, m.data() + c * nmodes, sizeof(cx<double>) * nk3,
-                                    sizeof(cx<double>) * nk3, (size_t)nk2 * nk1, hipMemcpyHostToDevice, st));
+        PackArgs p{};
+        for (int c = 0; c < 3; c++) p.padded[c] = f[c];
+        p.compact = (cx<double>*)X2;
+        p.row0 = (uint32_t)row0; p.nrow = (uint32_t)nrow; p.nk3 = (uint32_t)nk3; p.nk3p = (uint32_t)nk3p;
+        p.nk1 = nk1; p.nk2 = nk2;
+        p.notcubic = cfg.isNotCubic; p.Lx = cfg.Lx; p.Ly = cfg.Ly; p.Lz = cfg.Lz;
+        if (row0 < 0 || nrow < 0 || row0 + nrow > (int64_t)nk2 * nk1 || pack_bytes(nrow) > (size_t)9 * x2_slot * tsz)
+            throw Error(SPNS_EINVAL, "packed state exceeds its buffer");
+        return p;
+    }
+    size_t pack_bytes(int64_t nrow) const { return sizeof(cx<double>) * 3 * (size_t)nrow * nk3; }
+
+    // h: [3][nmodes] complex; modes masked by the length factors are zeroed
+    void upload_state(const void* h)
+    {
+        const int64_t rows = (int64_t)nk2 * nk1;
+        const PackArgs p = pack_args((void* const*)uk, 0, rows);
+        hcopy.copy(const_cast<void*>(h), p.compact, pack_bytes(rows), false, cfg.device, st);
+        HIPCHK(launch_unpack(p, st));
         reset_history();
     }
 
@@ -811,14 +925,13 @@ struct spns_ctx {
         write_scalars(s);
     }
 
-    std::vector<std::complex<double>> download_state(cx<double>* const* src)
+    // rows of three pitched fields into host memory, [3][nrow][nk3] complex FP64
+    void download(void* const* f, bool fp32, int64_t row0, int64_t nrow, void* out)
     {
-        std::vector<std::complex<double>> h(3 * (size_t)nmodes);
-        for (int c = 0; c < 3; c++)
-            HIPCHK(hipMemcpy2DAsync(h.data() + c * nmodes, sizeof(cx<double>) * nk3, src[c], sizeof(cx<double>) * nk3p,
-                                    sizeof(cx<double>) * nk3, (size_t)nk2 * nk1, hipMemcpyDeviceToHost, st));
-        HIPCHK(hipStreamSynchronize(st));
-        return h;
+        if (nrow == 0) return;
+        const PackArgs p = pack_args(f, row0, nrow);
+        HIPCHK(launch_pack(p, fp32, st));
+        hcopy.copy(out, p.compact, pack_bytes(nrow), true, cfg.device, st);
     }
 
     int64_t compact_index(int k1, int k2, int k3) const
@@ -982,7 +1095,7 @@ struct spns_batch {
             a.invy2.setflag = c->x1v;
         }
         a.invx = c->inv_x_args(false);
-        a.z = c->zpass_args(nullptr);
+        a.z = c->zpass_args();
         a.fwdx = c->fwd_x_args();
         a.fwdy = c->fwd_y_args(c->nfwd);
         a.epi = c->epi_args(EPI_STEP);
@@ -1109,11 +1222,13 @@ struct spns_batch {
     {
         if (s < 0 || s >= nslots || !slot[s]) throw Error(SPNS_EINVAL, "no context in this slot");
         spns_ctx* c = slot[s];
-        if (state)
-            for (int q = 0; q < 3; q++)
-                HIPCHK(hipMemcpy2DAsync(state + 2 * (size_t)q * c->nmodes, sizeof(cx<double>) * c->nk3, c->uk[q],
-                                        sizeof(cx<double>) * c->nk3p, sizeof(cx<double>) * c->nk3, (size_t)c->nk2 * c->nk1,
-                                        hipMemcpyDeviceToHost, st));
+        if (state) {
+            // packed on the batch's stream: the slot's X2 is free between chunks
+            const int64_t rows = (int64_t)c->nk2 * c->nk1;
+            const PackArgs p = c->pack_args((void* const*)c->uk, 0, rows);
+            HIPCHK(launch_pack(p, false, st));
+            HIPCHK(hipMemcpyAsync(state, p.compact, c->pack_bytes(rows), hipMemcpyDeviceToHost, st));
+        }
         if (ek) HIPCHK(hipMemcpyAsync(ek, c->ek, sizeof(double) * c->nbins, hipMemcpyDeviceToHost, st));
         HIPCHK(hipEventRecord(ev, st));
     }
@@ -1211,9 +1326,8 @@ int spns_set_state(spns_ctx* ctx, const double* state)
     API_BEGIN(ctx)
     ctx->x1_stale();  // the state changes
     if (!state) throw Error(SPNS_EINVAL, "null state");
-    std::vector<std::complex<double>> h(3 * (size_t)ctx->nmodes);
-    std::memcpy(h.data(), state, sizeof(double) * 6 * ctx->nmodes);
-    ctx->upload_state(h);
+    HIPCHK(hipSetDevice(ctx->cfg.device));
+    ctx->upload_state(state);
     API_END(ctx)
 }
 
@@ -1221,8 +1335,7 @@ int spns_get_state(spns_ctx* ctx, double* state)
 {
     API_BEGIN(ctx)
     if (!state) throw Error(SPNS_EINVAL, "null output");
-    auto h = ctx->download_state(ctx->uk);
-    std::memcpy(state, h.data(), sizeof(double) * 6 * ctx->nmodes);
+    ctx->download((void* const*)ctx->uk, false, 0, (int64_t)ctx->nk2 * ctx->nk1, state);
     API_END(ctx)
 }
 
@@ -1231,12 +1344,7 @@ int spns_get_state_planes(spns_ctx* ctx, int32_t i2_first, int32_t n_i2, double*
     API_BEGIN(ctx)
     if (!out || i2_first < 0 || n_i2 < 0 || (int64_t)i2_first + n_i2 > ctx->nk2)
         throw Error(SPNS_EINVAL, "i2 range outside the compact box");
-    const size_t plane = (size_t)ctx->nk1 * ctx->nk3;  // modes per i2 plane (compact)
-    for (int c = 0; c < 3; c++)
-        HIPCHK(hipMemcpy2DAsync(out + 2 * (size_t)c * n_i2 * plane, sizeof(cx<double>) * ctx->nk3,
-                                ctx->uk[c] + (size_t)i2_first * ctx->nk1 * ctx->nk3p, sizeof(cx<double>) * ctx->nk3p,
-                                sizeof(cx<double>) * ctx->nk3, (size_t)n_i2 * ctx->nk1, hipMemcpyDeviceToHost, ctx->st));
-    HIPCHK(hipStreamSynchronize(ctx->st));
+    ctx->download((void* const*)ctx->uk, false, (int64_t)i2_first * ctx->nk1, (int64_t)n_i2 * ctx->nk1, out);
     API_END(ctx)
 }
 
@@ -1244,22 +1352,8 @@ int spns_get_rhist(spns_ctx* ctx, double* rh)
 {
     API_BEGIN(ctx)
     if (!rh) throw Error(SPNS_EINVAL, "null output");
-    if (ctx->prec == PREC_FP64) {
-        auto h = ctx->download_state((cx<double>* const*)ctx->R);
-        std::memcpy(rh, h.data(), sizeof(double) * 6 * ctx->nmodes);
-    } else {
-        // FP32-split: the history is held in FP32; widened here
-        std::vector<cx<float>> h(3 * (size_t)ctx->nmodes);
-        for (int c = 0; c < 3; c++)
-            HIPCHK(hipMemcpy2DAsync(h.data() + c * ctx->nmodes, sizeof(cx<float>) * ctx->nk3, ctx->R[c],
-                                    sizeof(cx<float>) * ctx->nk3p, sizeof(cx<float>) * ctx->nk3, (size_t)ctx->nk2 * ctx->nk1,
-                                    hipMemcpyDeviceToHost, ctx->st));
-        HIPCHK(hipStreamSynchronize(ctx->st));
-        for (size_t i = 0; i < h.size(); i++) {
-            rh[2 * i] = h[i].x;
-            rh[2 * i + 1] = h[i].y;
-        }
-    }
+    // FP32-split: the history is held in FP32; the pack widens it
+    ctx->download(ctx->R, ctx->prec == PREC_FP32, 0, (int64_t)ctx->nk2 * ctx->nk1, rh);
     API_END(ctx)
 }
 
@@ -1333,7 +1427,7 @@ int spns_init_from_physical(spns_ctx* ctx, const double* u, const double* v, con
                 int64_t q = ctx->compact_index(k1, k2, k3);
                 for (int c = 0; c < 3; c++) h[c * ctx->nmodes + q] = spec[c][idf];
             }
-    ctx->upload_state(h);
+    ctx->upload_state(h.data());
     API_END(ctx)
 }
 
@@ -1369,7 +1463,7 @@ int spns_init_k41(spns_ctx* ctx, int32_t nranks)
                     }
                 }
     }
-    ctx->upload_state(h);
+    ctx->upload_state(h.data());
     HIPCHK(launch_ccc(ctx->shell_args(), ctx->st));  // src/HIT_LES.cpp:527
     std::vector<double> k41(ctx->last_rad + 1, 0.0);
     for (int K = 1; K <= ctx->last_rad; K++) k41[K] = std::pow(K, -5.0 / 3.0);
@@ -1407,7 +1501,7 @@ int spns_finish_init(spns_ctx* ctx, int32_t isReLambda)
     s.nu = ctx->cfg.nu;
     s.kappa = 0.5;
     ctx->write_scalars(s);
-    ctx->velocity_pass(nullptr);
+    ctx->velocity_pass();
     if (!isReLambda) HIPCHK(launch_finalize(ctx->fin_args(FIN_DT), ctx->st));
     ctx->reduce_state();
     HIPCHK(hipStreamSynchronize(ctx->st));
@@ -1513,7 +1607,7 @@ int spns_pass_kernels(spns_ctx* ctx, int32_t* zpass_kernel, int32_t* fused_epilo
 {
     API_BEGIN(ctx)
     if (zpass_kernel) {
-        ZArgs z = ctx->zpass_args(nullptr);
+        ZArgs z = ctx->zpass_args();
         z.kernel = ctx->zkernel;
         *zpass_kernel = zpass_kernel_of(ctx->Mz, ctx->prec, z);
     }
@@ -1529,37 +1623,41 @@ int spns_get_scalars(spns_ctx* ctx, spns_scalars* out)
     API_END(ctx)
 }
 
-// The velocity pass (current state) or the step-start pass into a device
-// buffer, then [c][y][x][z] copied out as [c][x][y][z] doubles.
+// The velocity pass (current state) or the step-start pass, exported by the z
+// pass as [x][y][z] doubles per component, then copied out.  The export goes
+// where the passes leave room (X2 beyond the three velocity fields, X1 once the
+// x pass has read it), and into memory of its own where they do not (long z).
 static void physical_out(spns_ctx* ctx, double* uvw, bool step_start)
 {
     if (!uvw) throw Error(SPNS_EINVAL, "null output");
-    const int Mx = ctx->Mx, My = ctx->My, Mz = ctx->Mz;
-    const size_t P = (size_t)Mx * My * Mz;
-    const size_t ts = ctx->prec == PREC_FP64 ? 8 : 4;
-    void* d = nullptr;
-    ctx->alloc(&d, 3 * P * ts);
+    HIPCHK(hipSetDevice(ctx->cfg.device));
+    const size_t P = (size_t)ctx->Mx * ctx->My * ctx->Mz, pb = sizeof(double) * P;
+    char* room[2] = {(char*)ctx->X2f(3), (char*)ctx->X1};
+    size_t left[2] = {(size_t)6 * ctx->x2_slot * ctx->tsz, (size_t)ctx->n_x1 * ctx->x1_slot * ctx->tsz};
+    double* d[3] = {};
+    void* own[3] = {};
     try {
-        if (step_start)
-            ctx->velocity_step_start(d);
-        else
-            ctx->velocity_pass(d);
-        std::vector<char> hbuf(3 * P * ts);
-        HIPCHK(hipMemcpyAsync(hbuf.data(), d, 3 * P * ts, hipMemcpyDeviceToHost, ctx->st));
-        HIPCHK(hipStreamSynchronize(ctx->st));
-        for (int c = 0; c < 3; c++)
-            for (int y = 0; y < My; y++)
-                for (int x = 0; x < Mx; x++)
-                    for (int z = 0; z < Mz; z++) {
-                        size_t s = c * P + ((size_t)y * Mx + x) * Mz + z;
-                        double v = ts == 8 ? ((double*)hbuf.data())[s] : (double)((float*)hbuf.data())[s];
-                        uvw[c * P + ((size_t)x * My + y) * Mz + z] = v;
-                    }
+        for (int c = 0; c < 3; c++) {
+            for (int r = 0; r < 2 && !d[c]; r++)
+                if (left[r] >= pb) {
+                    d[c] = (double*)room[r];
+                    room[r] += pb;
+                    left[r] -= pb;
+                }
+            if (!d[c]) {
+                ctx->alloc(&own[c], pb);
+                d[c] = (double*)own[c];
+            }
+        }
+        if (step_start) ctx->velocity_step_start(d);
+        else ctx->velocity_pass(d);
+        for (int c = 0; c < 3; c++) ctx->hcopy.copy(uvw + c * P, d[c], pb, true, ctx->cfg.device, ctx->st);
     } catch (...) {
-        hipFree(d);
+        hipStreamSynchronize(ctx->st);
+        for (void* p : own) hipFree(p);
         throw;
     }
-    hipFree(d);
+    for (void* p : own) hipFree(p);
 }
 
 int spns_velocity_physical(spns_ctx* ctx, double* uvw)
@@ -1596,7 +1694,7 @@ int spns_check_phys_four_energy(spns_ctx* ctx, double atol, double* ek_real, dou
 int spns_recalculate_velocity_antitransform(spns_ctx* ctx)
 {
     API_BEGIN(ctx)
-    ctx->velocity_pass(nullptr);
+    ctx->velocity_pass();
     API_END(ctx)
 }
 
@@ -1724,7 +1822,7 @@ int spns_profile_passes(spns_ctx* ctx, int32_t nsteps, double* ms)
             HIPCHK(hipEventRecord(ev[2], ctx->st));
             ctx->inv_x(false);
             HIPCHK(hipEventRecord(ev[3], ctx->st));
-            ctx->zpass(0, nullptr);
+            ctx->zpass(0);
             HIPCHK(hipEventRecord(ev[4], ctx->st));
             ctx->fwd_x();
             HIPCHK(hipEventRecord(ev[5], ctx->st));

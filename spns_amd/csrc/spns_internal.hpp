@@ -58,7 +58,8 @@ struct ZArgs {
     double Ax, Ay, Az;  // CFL divisors (src/HIT_LES.h:56-58)
     double ct;          // (C_Smag*delta)^2 (src/HIT_LES.cpp:132)
     double* z_partial;  // [gridDim.x][4]: MODE 0 sums of (du/dx)^2, (du/dx)^3; MODE 1 sum of u.u, 0; then the CFL maxima
-    void* phys;            // MODE 1: optional [3][npencil][L] physical export
+    double* phys[3];       // MODE 1: optional physical export of each component, [x][y][L]
+    int Mx, My;            // the export's extents (pencil = y Mx + x)
     const void* tw;
 };
 
@@ -123,6 +124,16 @@ struct ShellArgs {
     int notcubic, Lx, Ly, Lz;
     const double* ft;
     int last_eff, nullify;
+};
+
+// Compact box (the C ABI's [c][i2][i1][i3], FP64) to or from the pitched device
+// fields, rows [row0, row0 + nrow) of the (i2, i1) rows.
+struct PackArgs {
+    void* padded[3];  // cx<double>, or cx<float> (pack only: widened)
+    cx<double>* compact;  // [3][nrow][nk3]
+    uint32_t row0, nrow, nk3, nk3p;
+    int nk1, nk2;
+    int notcubic, Lx, Ly, Lz;  // unpack: modes masked by the length factors are zeroed
 };
 
 struct NormArgs {
@@ -190,6 +201,8 @@ hipError_t launch_finalize(const FinArgs& a, hipStream_t st, const BatchLaunch* 
 hipError_t launch_inv_spectra(int prec, const InvSpecArgs& a, int grid, double* out, hipStream_t st);
 hipError_t launch_set_left(int* left, const SlotSteps& s, int nslots, hipStream_t st);
 hipError_t launch_stream_copy(const void* in, void* out, int64_t bytes, int blocks, hipStream_t st);
+hipError_t launch_pack(const PackArgs& a, bool from_fp32, hipStream_t st);
+hipError_t launch_unpack(const PackArgs& a, hipStream_t st);
 hipError_t launch_forcing(const double* ek, const double* forced, double* ft, int last_eff, const ShellArgs& a, hipStream_t st);
 hipError_t launch_ccc(const ShellArgs& a, hipStream_t st);
 hipError_t launch_normalize(int prec, const NormArgs& a, hipStream_t st);
