@@ -25,6 +25,7 @@ UNITS = [
     ("spns_kernels.hip", "k2.o", ["-DSPNS_PART=2"]),
     ("spns_kernels.hip", "k3.o", ["-DSPNS_PART=3"]),
     ("spns_kernels.hip", "k4.o", ["-DSPNS_PART=4"]),
+    ("spns_kernels.hip", "k5.o", ["-DSPNS_PART=5"]),
     ("spns_ctx.hip", "ctx.o", []),
     ("hit.cpp", "hit.o", []),
     ("params.cpp", "params.o", []),

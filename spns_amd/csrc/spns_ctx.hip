@@ -222,7 +222,8 @@ struct spns_fft {
         a.tw = twx;
         int64_t cap = (int64_t)My * Mx * nk;
         check_strided(a, My, &cap, &cap, 0);
-        HIPCHK(launch_strided(Mx, prec, prec == PREC_FP64, prec == PREC_FP64, dir, a, My, st));
+        a.A = My;
+        HIPCHK(launch_line(Mx, prec, dir, a, st));
     }
     void fft_y(void* c, int dir)
     {
@@ -235,14 +236,13 @@ struct spns_fft {
         a.tw = twy;
         int64_t cap = (int64_t)My * Mx * nk;
         check_strided(a, 1, &cap, &cap, 0);
-        HIPCHK(launch_strided(My, prec, prec == PREC_FP64, prec == PREC_FP64, dir, a, 1, st));
+        a.A = 1;
+        HIPCHK(launch_line(My, prec, dir, a, st));
     }
     void z(const void* in, void* out, int dir)
     {
-        ZPlainArgs a{in, out, Mx, My, twz};
-        int64_t np = (int64_t)Mx * My;
-        int grid = (int)std::min<int64_t>((np + 1) / 2, 65536);
-        HIPCHK(launch_zplain(Mz, prec, dir, a, grid, st));
+        const ZPlainArgs a{in, out, Mx, My, twz};
+        HIPCHK(launch_zplain(Mz, prec, dir, a, st));
     }
 };
 

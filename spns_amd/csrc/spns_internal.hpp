@@ -188,7 +188,8 @@ hipError_t launch_strided(int L, int prec, int in_fp64, int out_fp64, int dir, c
 hipError_t launch_zpass(int L, int prec, int mode, const ZArgs& a, int grid, hipStream_t st, const BatchLaunch* bl = nullptr);
 int zpass_grid(int L, int prec, const ZArgs& a, int64_t npen);  // < 0: no such length / HIP error
 int zpass_kernel(int L, int prec, const ZArgs& a);              // kernel launch_zpass picks
-hipError_t launch_zplain(int L, int prec, int dir, const ZPlainArgs& a, int grid, hipStream_t st);
+hipError_t launch_zplain(int L, int prec, int dir, const ZPlainArgs& a, hipStream_t st);
+hipError_t launch_line(int L, int prec, int dir, const StridedArgs& a, hipStream_t st);  // in place, unpruned, any row alignment
 // inv: the variant with the next step's inverse y pass (k_yepi_inv), which
 // launch_yepi runs when ia (the inverse pass's arguments) is given; it sets
 // *x1v

@@ -165,16 +165,22 @@ __host__ __device__ constexpr bool sstage_fits()
 // i k transform of column b - TB, both formed from one staged tile), so the
 // next item's copy is issued after the one shared stage 0 and stays in
 // flight across both transforms; 2 the single jobs.
-template <typename TIN, typename TOUT, typename T, int L, int TB, int NT, int DIR, bool STDP = false, int JSEL = 0>
+// LINE: the unpruned in-place transform of the FFT_package layouts, whose rows
+// have no pitch: every staged column is checked against B (nothing outside the
+// rows is read), FP32 rows are copied 4 bytes a lane (an odd number of 8-byte
+// elements leaves them 8-byte aligned), and every twiddle factor is read from
+// the table.  An item's outputs are its own columns, which no other item reads,
+// so in place is safe with the next item's copy in flight.
+template <typename TIN, typename TOUT, typename T, int L, int TB, int NT, int DIR, bool STDP = false, int JSEL = 0, bool LINE = false>
 __device__ __forceinline__ void sstage_body(const StridedArgs& a)
 {
     constexpr int NB = JSEL == 1 ? 2 * TB : TB;  // columns of the transform (and LDS row pitch of fbuf)
     static_assert((TB & (TB - 1)) == 0, "column tile must be a power of two");
-    constexpr int SROWS = sstage_rows<L, DIR>();
-    constexpr int SPR = TB * (int)sizeof(cx<TIN>) / 16;  // 16-byte copy slots per staged row
-    constexpr int EPS = 16 / (int)sizeof(cx<TIN>);        // input elements per slot
+    constexpr int SROWS = LINE ? L : sstage_rows<L, DIR>();
+    constexpr int SLOT = LINE && sizeof(cx<TIN>) < 16 ? 4 : 16;  // bytes per lane of a copy
+    constexpr int SPR = TB * (int)sizeof(cx<TIN>) / SLOT;        // copy slots per staged row
     constexpr int NW = NT / 64;
-    constexpr int TWM = sizeof(T) == 8 ? 1 : 2;
+    constexpr int TWM = LINE ? 0 : sizeof(T) == 8 ? 1 : 2;
     constexpr int TWN = fft_twiddle_span<L, TWM>();  // the table entries the transform reads
     __shared__ __align__(16) cx<T> fbuf[L * NB];
     __shared__ __align__(16) cx<TIN> stg[SROWS * TB];
@@ -198,9 +204,6 @@ __device__ __forceinline__ void sstage_body(const StridedArgs& a)
     const int G = gridDim.x;  // a multiple of 8
     const int64_t lin = (int64_t)(blockIdx.x % 8) * (G / 8) + blockIdx.x / 8;
 
-    for (int i = t; i < TWN; i += NT) twl[i] = ((const cx<T>*)a.tw)[i];
-    __syncthreads();
-
     const int wave = __builtin_amdgcn_readfirstlane(t >> 6), lane = t & 63;
     const uint32_t stg_base = lds_addr(stg);
     const int nslot = a.nin * SPR;
@@ -209,16 +212,23 @@ __device__ __forceinline__ void sstage_body(const StridedArgs& a)
         const int r = (int)(it - ai * per_a);
         const int js = r / ntiles, b0 = (r - js * ntiles) * TB;
         const int jb = (int)((jsel >> (4 * js)) & 15);
-        const cx<TIN>* in = (const cx<TIN>*)a.job[jb].in + ai * a.in_a_stride + b0;
+        const char* in = (const char*)((const cx<TIN>*)a.job[jb].in + ai * a.in_a_stride + b0);
+        const int64_t rowb = a.in_row_stride * (int64_t)sizeof(cx<TIN>);
+        const int colb = LINE ? (a.B - b0) * (int)sizeof(cx<TIN>) : 0;  // bytes of this tile's rows
         for (int m = wave; m * 64 < nslot; m += NW) {
             const int s = m * 64 + lane;
             const int row = s / SPR, part = s - row * SPR;
-            if (s < nslot) dma16(in + (int64_t)row * a.in_row_stride + part * EPS, stg_base + (uint32_t)m * 1024u);
+            if (s < nslot && (!LINE || part * SLOT < colb)) {
+                const char* g = in + row * rowb + part * SLOT;
+                if constexpr (SLOT == 4) dma4(g, stg_base + (uint32_t)m * 256u);
+                else dma16(g, stg_base + (uint32_t)m * 1024u);
+            }
         }
     };
 
     int64_t it = lin;
-    if (it < nitems) issue(it);
+    if (it < nitems) issue(it);  // in flight while the twiddles are read
+    for (int i = t; i < TWN; i += NT) twl[i] = ((const cx<T>*)a.tw)[i];
     dma_wait();
     lds_barrier();
     for (; it < nitems; it += G) {
@@ -313,6 +323,16 @@ template <typename TIN, typename TOUT, typename T, int L, int TB, int NT, int DI
 __global__ __launch_bounds__(NT) void k_sstage(StridedArgs a)
 {
     sstage_body<TIN, TOUT, T, L, TB, NT, DIR, STDP, JSEL>(a);
+}
+
+// In-place transforms of the FFT_package drop-in along y or x.  Bounded by HBM
+// (one read and one write of the field).  The direct-load kernel it replaces
+// left the memory idle while a block transformed: 768^3 FP64 2.58 -> 2.07 ms
+// (3.5 TB/s), 384^3 FP32 353 -> 132 us a pass.
+template <typename T, int L, int TB, int NT, int DIR>
+__global__ __launch_bounds__(NT) void k_line(StridedArgs a)
+{
+    sstage_body<T, T, T, L, TB, NT, DIR, false, 0, true>(a);
 }
 
 template <typename TIN, typename TOUT, typename T, int L, int TB, int NT, int DIR, bool STDP = false, int JSEL = 0>
@@ -1288,68 +1308,108 @@ __global__ __launch_bounds__(256) void k_zwave(ZArgs a)
 // Plain z transforms for the FFT_package drop-in (reference layouts):
 //   c2r: complex [y][x][nk] -> real [x][y][2nk] padded (src/util.h:75-80)
 //   r2c: real [x][y][2nk] -> complex [y][x][nk]
-// Two pencils per block iteration are paired into one complex transform.
+// Two pencils are paired into one complex transform, NB pairs at a time.
+// Bounded by HBM (one read and one write of the field); every global access
+// runs along z, and the exchanges through LDS ([row][NB + 1]: an odd pitch, so
+// accesses along z spread over the banks) keep it so on both sides.  One pair
+// per 64-thread block, as before, left 56 of 64 lanes idle at L = 48 and wrote
+// the c2r's results 8 bytes at a time: 768^3 FP64 c2r 1.99 -> 1.63 ms, r2c 1.62 ->
+// 1.55 ms (4.7 TB/s), 384^3 FP32 122 -> 100 us.  Loads that wait for each other
+// in a loop cost more than either: 4.1 ms for the r2c.
 // ---------------------------------------------------------------------------
-template <typename T, int L, int NT, int DIR>
-__global__ __launch_bounds__(NT) void k_zplain(ZPlainArgs a)
+// Pairs per block: 8 at most, fewer where the exchange buffer would leave room
+// for less than three blocks per CU.
+template <typename T, int L>
+__host__ __device__ constexpr int zline_nb()
 {
-    __shared__ cx<T> lds[L];
-    const cx<T>* tw = (const cx<T>*)a.tw;
-    const int nk = L / 2 + 1;
-    const int64_t np = (int64_t)a.Mx * a.My;
-    for (int64_t pp = blockIdx.x; 2 * pp < np; pp += gridDim.x) {
-        const int64_t p0 = 2 * pp, p1 = 2 * pp + 1;
-        const bool has1 = p1 < np;
-        // pencil index p -> (y = p / Mx, x = p % Mx)
-        const int64_t y0 = p0 / a.Mx, x0 = p0 % a.Mx, y1 = p1 / a.Mx, x1 = p1 % a.Mx;
-        if (DIR > 0) {
-            const cx<T>* in = (const cx<T>*)a.in;
-            auto ld = [&](int64_t y, int64_t x, int k) { return in[(y * a.Mx + x) * nk + k]; };
-            auto load = [&](int b, int p) -> cx<T> {
-                (void)b;
-                cx<T> A, B = cx<T>{(T)0, (T)0};
-                if (p == 0 || (p == L / 2)) {
-                    A = ld(y0, x0, p);
-                    if (has1) B = ld(y1, x1, p);
-                    return cx<T>{A.x, B.x};
+    constexpr size_t el = sizeof(cx<T>) * L;
+    return L <= 144 ? 8 : el * 5 <= 40960 ? 4 : 2;
+}
+
+template <typename T, int L, int NB, int NT, int DIR>
+__global__ __launch_bounds__(NT) void k_zline(ZPlainArgs a)
+{
+    constexpr int LD = NB + 1, nk = L / 2 + 1;
+    constexpr int NIT = (NB * nk + NT - 1) / NT;
+    __shared__ __align__(16) cx<T> fbuf[L * LD];
+    __shared__ __align__(16) cx<T> twl[L];
+    const int t = threadIdx.x;
+    const uint32_t Mx = a.Mx, My = a.My, np = Mx * My;
+    // pencil p = y Mx + x: offset of its real row
+    auto real_row = [&](uint32_t p) -> int64_t {
+        const uint32_t y = p / Mx;
+        return ((int64_t)(p - y * Mx) * My + y) * (2 * nk);
+    };
+    auto store_lds = [&](int b, int p, cx<T> v) { fbuf[p * LD + b] = v; };
+    auto none = [] {};
+    bool first = true;
+    for (uint32_t q0 = blockIdx.x * NB; 2 * q0 < np; q0 += gridDim.x * NB) {  // first pair of the group
+        if constexpr (DIR > 0) {
+            const cx<T>* __restrict__ in = (const cx<T>*)a.in;
+            T* __restrict__ out = (T*)a.out;
+            // every load of the group is in flight before the first is used
+            cx<T> A[NIT], B[NIT];
+#pragma unroll
+            for (int i = 0; i < NIT; i++) {
+                const int idx = t + i * NT, b = idx / nk, k = idx - b * nk;
+                const uint32_t p0 = 2 * (q0 + b);
+                const bool ok = idx < NB * nk;
+                A[i] = ok && p0 < np ? in[(int64_t)p0 * nk + k] : cx<T>{(T)0, (T)0};
+                B[i] = ok && p0 + 1 < np ? in[(int64_t)(p0 + 1) * nk + k] : cx<T>{(T)0, (T)0};
+            }
+            if (first)
+                for (int i = t; i < L; i += NT) twl[i] = ((const cx<T>*)a.tw)[i];
+            lds_barrier();  // the previous group's reads are done
+#pragma unroll
+            for (int i = 0; i < NIT; i++) {
+                const int idx = t + i * NT, b = idx / nk, k = idx - b * nk;
+                if (idx < NB * nk) {
+                    if (k == 0 || 2 * k == L) {
+                        fbuf[k * LD + b] = cx<T>{A[i].x, B[i].x};  // only the real part of the end terms enters
+                    } else {
+                        fbuf[k * LD + b] = cx<T>{A[i].x - B[i].y, A[i].y + B[i].x};
+                        fbuf[(L - k) * LD + b] = cx<T>{A[i].x + B[i].y, B[i].x - A[i].y};
+                    }
                 }
-                if (p < nk) {
-                    A = ld(y0, x0, p);
-                    if (has1) B = ld(y1, x1, p);
-                    return cx<T>{A.x - B.y, A.y + B.x};
-                }
-                const int k = L - p;
-                A = ld(y0, x0, k);
-                if (has1) B = ld(y1, x1, k);
-                return cx<T>{A.x + B.y, B.x - A.y};
-            };
-            T* out = (T*)a.out;
-            auto store = [&](int b, int p, cx<T> v) {
-                (void)b;
-                out[(x0 * a.My + y0) * 2 * nk + p] = v.x;
-                if (has1) out[(x1 * a.My + y1) * 2 * nk + p] = v.y;
-            };
-            Fft<T, L, 1, NT, 1, +1>::run(lds, tw, load, store);
+            }
+            auto load_lds = [&](int b, int p) -> cx<T> { return fbuf[p * LD + b]; };
+            FftS<T, L, NB, NT, LD, +1, true, 0>::template run<true>(fbuf, twl, load_lds, store_lds, none, t);
+            lds_barrier();
+            for (int idx = t; idx < NB * L; idx += NT) {
+                const int b = idx / L, n = idx - b * L;
+                const uint32_t p0 = 2 * (q0 + b);
+                const cx<T> v = fbuf[n * LD + b];
+                if (p0 < np) out[real_row(p0) + n] = v.x;
+                if (p0 + 1 < np) out[real_row(p0 + 1) + n] = v.y;
+            }
         } else {
-            const T* in = (const T*)a.in;
+            const T* __restrict__ in = (const T*)a.in;
+            cx<T>* __restrict__ out = (cx<T>*)a.out;
+            // stage 0 reads its inputs itself, consecutive threads along z
             auto load = [&](int b, int p) -> cx<T> {
-                (void)b;
-                T re = in[(x0 * a.My + y0) * 2 * nk + p];
-                T im = has1 ? in[(x1 * a.My + y1) * 2 * nk + p] : (T)0;
-                return cx<T>{re, im};
+                const uint32_t p0 = 2 * (q0 + b);
+                cx<T> v = cx<T>{(T)0, (T)0};
+                if (p0 < np) v.x = in[real_row(p0) + p];
+                if (p0 + 1 < np) v.y = in[real_row(p0 + 1) + p];
+                return v;
             };
-            auto store = [&](int b, int p, cx<T> v) { (void)b; lds[p] = v; };
-            Fft<T, L, 1, NT, 1, -1>::run(lds, tw, load, store);
-            __syncthreads();
-            cx<T>* out = (cx<T>*)a.out;
-            for (int k = threadIdx.x; k < nk; k += NT) {
-                const cx<T> Z = lds[k], Zc = lds[(L - k) % L];
+            if (first)
+                for (int i = t; i < L; i += NT) twl[i] = ((const cx<T>*)a.tw)[i];
+            // SYNC0: a barrier between stage 0's reads and its writes, which
+            // the previous group's unpack must have left
+            FftS<T, L, NB, NT, LD, -1, true, 0, true>::template run<false>(fbuf, twl, load, store_lds, none, t);
+            lds_barrier();
+            for (int idx = t; idx < NB * nk; idx += NT) {
+                const int b = idx / nk, k = idx - b * nk;
+                const uint32_t p0 = 2 * (q0 + b);
+                if (p0 >= np) continue;
+                const cx<T> Z = fbuf[k * LD + b], Zc = fbuf[(k == 0 ? 0 : L - k) * LD + b];
                 const T h = (T)0.5;
-                out[(y0 * a.Mx + x0) * nk + k] = cx<T>{h * (Z.x + Zc.x), h * (Z.y - Zc.y)};
-                if (has1) out[(y1 * a.Mx + x1) * nk + k] = cx<T>{h * (Z.y + Zc.y), h * (Zc.x - Z.x)};
+                out[(int64_t)p0 * nk + k] = cx<T>{h * (Z.x + Zc.x), h * (Z.y - Zc.y)};
+                if (p0 + 1 < np) out[(int64_t)(p0 + 1) * nk + k] = cx<T>{h * (Z.y + Zc.y), h * (Zc.x - Z.x)};
             }
         }
-        __syncthreads();
+        first = false;
     }
 }
 
@@ -2529,28 +2589,73 @@ hipError_t launch_zpass(int L, int prec, int mode, const ZArgs& a, int grid, hip
 
 #endif
 
-#if SPNS_PART == 0 || SPNS_PART == 4
-template <typename T, int L, int DIR>
-static hipError_t launch_zplain_L(const ZPlainArgs& a, int grid, hipStream_t st)
+#if SPNS_PART == 0 || SPNS_PART == 5
+// Persistent grid of a kernel: as many blocks as fit the device, at most items,
+// rounded up to the 8 XCDs; -1 on an error.
+template <class Kern>
+static int resident_grid(Kern kern, int nt, int64_t items)
 {
-    constexpr int NT = 64;
-    hipLaunchKernelGGL((k_zplain<T, L, NT, DIR>), dim3(grid), dim3(NT), 0, st, a);
+    int nb = 0, dev = 0, ncu = 0;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, kern, nt, 0) != hipSuccess || nb < 1) nb = 1;
+    if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return -1;
+    int64_t g = (int64_t)ncu * nb;
+    if (items < g) g = items;
+    return (int)((g + 7) / 8 * 8);
+}
+
+template <typename T, int L, int DIR>
+static hipError_t launch_zline_L(const ZPlainArgs& a, hipStream_t st)
+{
+    constexpr int NB = zline_nb<T, L>(), NT = sstage_nt<L, NB>();
+    const int64_t np = (int64_t)a.Mx * a.My;
+    if (np >= ((int64_t)1 << 30)) return hipErrorInvalidValue;  // 32-bit pencil index
+    const int g = resident_grid(k_zline<T, L, NB, NT, DIR>, NT, ((np + 1) / 2 + NB - 1) / NB);
+    if (g < 1) return hipErrorUnknown;
+    hipLaunchKernelGGL((k_zline<T, L, NB, NT, DIR>), dim3(g), dim3(NT), 0, st, a);
     return hipGetLastError();
 }
 
-hipError_t launch_zplain(int L, int prec, int dir, const ZPlainArgs& a, int grid, hipStream_t st)
+hipError_t launch_zplain(int L, int prec, int dir, const ZPlainArgs& a, hipStream_t st)
 {
 #define X(LL)                                                                                        \
     if (L == LL) {                                                                                   \
-        if (prec == PREC_FP64) return dir > 0 ? launch_zplain_L<double, LL, +1>(a, grid, st)         \
-                                              : launch_zplain_L<double, LL, -1>(a, grid, st);        \
-        return dir > 0 ? launch_zplain_L<float, LL, +1>(a, grid, st) : launch_zplain_L<float, LL, -1>(a, grid, st); \
+        if (prec == PREC_FP64) return dir > 0 ? launch_zline_L<double, LL, +1>(a, st)                \
+                                              : launch_zline_L<double, LL, -1>(a, st);               \
+        return dir > 0 ? launch_zline_L<float, LL, +1>(a, st) : launch_zline_L<float, LL, -1>(a, st); \
     }
     SPNS_FOR_EACH_L(X)
 #undef X
     return hipErrorInvalidValue;
 }
 
+template <typename T, int L, int DIR>
+static hipError_t launch_line_L(const StridedArgs& a, hipStream_t st)
+{
+    constexpr int TB = strided_tb<T, L>(), NT = sstage_nt<L, TB>();
+    static_assert(sizeof(cx<T>) * (2 * (size_t)L * TB + L) <= 160 * 1024 - 512, "tile, staging and table fit the LDS");
+    if (a.njobs != 1 || a.nin != L || a.nout != L || a.job[0].out2 || a.job[0].deriv) return hipErrorInvalidValue;
+    const int g = resident_grid(k_line<T, L, TB, NT, DIR>, NT, (int64_t)a.A * ((a.B + TB - 1) / TB));
+    if (g < 1) return hipErrorUnknown;
+    hipLaunchKernelGGL((k_line<T, L, TB, NT, DIR>), dim3(g), dim3(NT), 0, st, a);
+    return hipGetLastError();
+}
+
+hipError_t launch_line(int L, int prec, int dir, const StridedArgs& a, hipStream_t st)
+{
+#define X(LL)                                                                                        \
+    if (L == LL) {                                                                                   \
+        if (prec == PREC_FP64) return dir > 0 ? launch_line_L<double, LL, +1>(a, st)                 \
+                                              : launch_line_L<double, LL, -1>(a, st);                \
+        return dir > 0 ? launch_line_L<float, LL, +1>(a, st) : launch_line_L<float, LL, -1>(a, st);  \
+    }
+    SPNS_FOR_EACH_L(X)
+#undef X
+    return hipErrorInvalidValue;
+}
+
+#endif
+
+#if SPNS_PART == 0 || SPNS_PART == 4
 
 // ---------------------------------------------------------------------------
 // Shell spectra of the five velocity-gradient invariants (src/HIT_LES.cpp:
