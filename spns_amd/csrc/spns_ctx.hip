@@ -421,6 +421,7 @@ struct spns_ctx {
             zq.pitch = nk3p;
             zq.nk3 = nk3;
             zq.les = les;
+            zq.npencil = npen;
             grid_z = zpass_grid(Mz, prec, zq, npen);
             if (grid_z <= 0) throw Error(SPNS_EHIP, "z pass: no launch configuration for this length");
         }

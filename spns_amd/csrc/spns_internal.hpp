@@ -186,6 +186,8 @@ hipError_t launch_strided_fp32(int L, int in_fp64, int dir, const StridedArgs& a
 hipError_t launch_strided(int L, int prec, int in_fp64, int out_fp64, int dir, const StridedArgs& a, int A, hipStream_t st,
                           const BatchLaunch* bl = nullptr);
 hipError_t launch_zpass(int L, int prec, int mode, const ZArgs& a, int grid, hipStream_t st, const BatchLaunch* bl = nullptr);
+hipError_t launch_zreg(int L, int prec, const ZArgs& a, int grid, hipStream_t st, const BatchLaunch* bl);  // k_zreg, where launch_zpass picks it
+int zreg_blocks(int L, int prec, bool les);                                                                 // its blocks per CU
 int zpass_grid(int L, int prec, const ZArgs& a, int64_t npen);  // < 0: no such length / HIP error
 int zpass_kernel(int L, int prec, const ZArgs& a);              // kernel launch_zpass picks
 hipError_t launch_zplain(int L, int prec, int dir, const ZPlainArgs& a, hipStream_t st);

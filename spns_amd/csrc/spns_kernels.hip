@@ -1154,6 +1154,359 @@ __global__ __launch_bounds__(NT) void k_zfuse_b(const ZArgs* __restrict__ arr, c
 }
 
 // ---------------------------------------------------------------------------
+// z pass with the next pencils' inputs held in registers (the default at the
+// standard 3/2 padding for every LES and for DNS below L = 768).
+// A block takes PP pencils at a time.  Each thread holds its share of their
+// spectra (pair column b, k3 = k), loaded one group ahead, and spreads it into
+// the pair buffer as Z[k] and Z[L - k]; nothing is staged in LDS, and what the
+// pairing costs is paid once per (k, column) instead of once per transform
+// input.  The buffer's columns are c PP + pp (pair c of pencil pp), so each
+// point's products stay in that point's own columns.
+//   LES: 6 PP inverse columns, products in place, 5 PP forward columns.
+//   DNS: one transform of 8 PP columns; the last 2 PP are the products of the
+//   previous group, run forward as conj(inverse(conj x)) (as k_zfuse does).
+// What bounds it: LDS and the latency between barriers in FP64 (so the room the
+// staging area took goes to more blocks per CU), vector-ALU issue in FP32 at
+// short lengths (so PP is taken to fill whole waves with butterflies).
+// z pass, one run: 256^3 LES 2.93 -> 2.34 ms FP64, 1.43 -> 1.18 FP32; 192^3 DNS
+// FP64 1.01 -> 0.66; 128^3 DNS FP64 243 -> 181 us; 16 x 64^3 DNS FP32 359 -> 261 us.
+// ---------------------------------------------------------------------------
+// Pair (A, B) at k3 = k: Z[k] (lo) and Z[L - k] (hi) of A + i B; dza / dzb: the
+// field is d_z of the one read.  Only the real part of k3 = 0 enters (as in a
+// c2r).  Products are rounded before the sums, as in every loader of these pairs.
+template <typename T>
+__device__ __forceinline__ void z_pair(cx<T> A, cx<T> B, int k, bool dza, bool dzb, cx<T>& lo, cx<T>& hi)
+{
+#pragma clang fp contract(off)
+    const T kk = (T)k;
+    if (dza) A = cx<T>{-kk * A.y, kk * A.x};
+    if (dzb) B = cx<T>{-kk * B.y, kk * B.x};
+    if (k == 0) A.y = B.y = (T)0;
+    lo = cx<T>{A.x - B.y, A.y + B.x};
+    hi = cx<T>{A.x + B.y, B.x - A.y};
+}
+
+// (f, d_z f) = (1 - k) f and (1 + k) conj f
+template <typename T>
+__device__ __forceinline__ void z_pair_dz(cx<T> A, int k, cx<T>& lo, cx<T>& hi)
+{
+#pragma clang fp contract(off)
+    const T a = (T)1 - (T)k, b = (T)1 + (T)k;
+    if (k == 0) A.y = (T)0;
+    lo = cx<T>{a * A.x, a * A.y};
+    hi = cx<T>{b * A.x, b * -A.y};
+}
+
+// Pencils per block: whole waves of butterflies at the short lengths.
+template <int L, bool LES>
+__host__ __device__ constexpr int zreg_pp()
+{
+    return LES ? 1 : L <= 72 ? 4 : L <= 144 ? 2 : 1;
+}
+
+// Threads: one butterfly each in every stage after the first (whose radix is
+// small where it has more), and one point each (an LES holds the products of a
+// thread's points in registers: two of them cost 208 us against 134 at 144, FP64).
+template <int L, int NB>
+__host__ __device__ constexpr int zreg_nt(int points)
+{
+    int m = points > 64 ? points : 64;
+    for (int s = 1; s < Plan<L>::n; s++) {
+        const int b = (L / Plan<L>::r(s)) * NB;
+        m = b > m ? b : m;
+    }
+    if (Plan<L>::r(0) > 4 && (L / Plan<L>::r(0)) * NB > m) m = (L / Plan<L>::r(0)) * NB;
+    m = (m + 63) / 64 * 64;
+    return m > 1024 ? 1024 : m;
+}
+
+// DNS pairs each velocity component with its own d_z where k_zfuse's
+// compile-time loader did (L / R0 = 64 or 128), else the logical fields in order.
+template <int L, bool LES>
+__host__ __device__ constexpr bool zreg_dzpair()
+{
+    return !LES && (L / Plan<L>::r(0) == 64 || L / Plan<L>::r(0) == 128);
+}
+
+template <typename T, int L, bool LES>
+struct ZReg {
+    static constexpr int PP = zreg_pp<L, LES>();
+    static constexpr int NI = 6 * PP, NF = (LES ? 5 : 2) * PP;
+    static constexpr int NB = LES ? NI : NI + NF;
+    static constexpr int NT = zreg_nt<L, NB>(LES ? PP * L : 0);
+    // row pitch: LES columns are packed (consecutive butterflies then read
+    // consecutive elements), the products repacked to their five columns; the
+    // DNS's eight would put a column's rows on the same banks
+    static constexpr int LD = LES ? NB : NB + 1;
+    static constexpr int LDF = LES ? NF : LD;
+    static constexpr int NKC = L / 3 + 1;
+    static constexpr int TWM = sizeof(T) == 8 ? 1 : 2;
+    static constexpr size_t lds = sizeof(cx<T>) * ((size_t)L * LD + fft_twiddle_span<L, TWM>()) + 9 * sizeof(void*);
+    static constexpr bool fits = L % 3 == 0 && lds <= 160 * 1024 - 512;
+    static constexpr int waves = (int)((160 * 1024) / lds) * (NT / 64) / 4;  // per SIMD, by LDS
+    static constexpr int W = waves < 1 ? 1 : waves > 4 ? 4 : waves;
+};
+
+// k_zreg for DNS: below L = 768, where k_zfuse has its swizzled layout, and not
+// for FP32 at 288 and 384, where k_zfuse's three blocks per CU keep the vector
+// ALU busier (0.373 against 0.405 ms at 192^3, 0.779 against 0.858 at 256^3).
+template <typename T, int L>
+constexpr bool zreg_dns()
+{
+    return L < 768 && !(sizeof(T) == 4 && (L == 288 || L == 384)) && ZReg<T, L, false>::fits;
+}
+
+template <typename T, int L, bool LES>
+__device__ __forceinline__ void zreg_body(const ZArgs& a)
+{
+    using Z = ZReg<T, L, LES>;
+    constexpr int PP = Z::PP, NI = Z::NI, NF = Z::NF, NB = Z::NB, NT = Z::NT, LD = Z::LD, LDF = Z::LDF, NKC = Z::NKC, TWM = Z::TWM;
+    constexpr int NITEM = NI * NKC, NIT = (NITEM + NT - 1) / NT;
+    constexpr int TWN = fft_twiddle_span<L, TWM>();
+    constexpr bool DZP = zreg_dzpair<L, LES>();
+    // What a thread keeps across the loop instead of recomputing it per group: in
+    // a DNS its items' indices and source pointers, in an FP64 LES the pointers.
+    // (FP32 LES at 384: 1.39 ms with the pointers kept, 1.19 without: 64 VGPRs.)
+    constexpr bool HOIST = !LES || sizeof(T) == 8, HOISTI = !LES;
+    static_assert(sizeof(cx<T>) * L * LD >= 6 * (NT / 64) * sizeof(double), "reduction scratch aliases the pair buffer");
+    __shared__ __align__(16) cx<T> fbuf[L * LD];
+    __shared__ __align__(16) cx<T> twl[TWN];
+    __shared__ cx<T>* fld[9];
+    const int t = threadIdx.x;
+    const int pitch = a.pitch;
+    T mu = (T)0, mv = (T)0, mw = (T)0;
+    double vmax_sa = 0.0, s2 = 0.0, s3 = 0.0;
+    const double iAx = a.Ax, iAy = a.Ay, iAz = a.Az;
+    const bool sa = a.sa;
+    if (t < 9) fld[t] = (cx<T>*)a.f[t];
+    __syncthreads();
+
+    // logical pairs in order: see k_zstage; with DZP pair c < 3 is (f_c, d_z f_c),
+    // c >= 3 (d_x, d_y) of component c - 3
+    constexpr uint32_t SRC_A = DZP ? 0x543210u : 0x814620u, SRC_B = DZP ? 0x876000u : 0x257031u;
+    constexpr uint32_t DZ_A = DZP ? 0u : 0x10u, DZ_B = DZP ? 0u : 0x24u;
+    // this thread's items: column, k3 and where the two spectra lie (global
+    // loads: a pointer read from LDS would make them flat ones, which the
+    // LDS-only barriers wait for)
+    typedef const __attribute__((address_space(1))) cx<T>* gptr;
+    const int64_t step = (int64_t)gridDim.x * PP * pitch;  // a group's pencils to the next group's
+    cx<T> A[NIT], B[NIT];
+    auto item = [&](int i, int tl, int& col, int& c, int& k) -> bool {
+        const int idx = tl + i * NT;
+        col = idx / NKC;
+        k = idx - col * NKC;
+        c = col / PP;
+        return (i + 1) * NT <= NITEM || idx < NITEM;
+    };
+    // source pointer of an item's two spectra in the group at pen0
+    auto src = [&](uint32_t tab, int col, int c, int k, int64_t pen0) -> gptr {
+        return (gptr)fld[(tab >> (4 * c)) & 15] + (pen0 + (col - c * PP)) * pitch + k;
+    };
+    gptr ga[HOIST ? NIT : 1], gb[HOIST ? NIT : 1];
+#pragma unroll
+    for (int i = 0; i < NIT; i++) {
+        A[i] = B[i] = cx<T>{(T)0, (T)0};
+        if constexpr (HOIST) {
+            int col, c, k;
+            if (!item(i, t, col, c, k)) col = c = k = 0;
+            ga[i] = src(SRC_A, col, c, k, (int64_t)blockIdx.x * PP);
+            gb[i] = src(SRC_B, col, c, k, (int64_t)blockIdx.x * PP);
+        }
+    }
+    // loads the group at pen0 (with HOIST the one the pointers are at, and
+    // moves them on to the next)
+    auto fetch = [&](int64_t pen0, int tl) {
+#pragma unroll
+        for (int i = 0; i < NIT; i++) {
+            int col, c, k;
+            if (item(i, tl, col, c, k)) {
+                const gptr pa = HOIST ? ga[HOIST ? i : 0] : src(SRC_A, col, c, k, pen0);
+                A[i].x = pa->x, A[i].y = pa->y;
+                if (!DZP || c >= 3) {
+                    const gptr pb = HOIST ? gb[HOIST ? i : 0] : src(SRC_B, col, c, k, pen0);
+                    B[i].x = pb->x, B[i].y = pb->y;
+                }
+            }
+            if constexpr (HOIST) {
+                ga[i] += step;
+                gb[i] += step;
+            }
+        }
+    };
+    auto spread = [&](int tl) {
+#pragma unroll
+        for (int i = 0; i < NIT; i++) {
+            int col, c, k;
+            if (item(i, tl, col, c, k)) {
+                cx<T> lo, hi;
+                if (DZP && c < 3) z_pair_dz(A[i], k, lo, hi);
+                else z_pair(A[i], B[i], k, (DZ_A >> c) & 1, (DZ_B >> c) & 1, lo, hi);
+                fbuf[k * LD + col] = lo;
+                if (k > 0) fbuf[(L - k) * LD + col] = hi;
+            }
+        }
+        if constexpr (!LES) {
+            // the zero padding (an LES's loader skips it)
+            constexpr int GAP = L - 2 * NKC + 1;
+            for (int idx = tl; idx < GAP * NI; idx += NT) {
+                const int r = idx / NI;
+                fbuf[(NKC + r) * LD + (idx - r * NI)] = cx<T>{(T)0, (T)0};
+            }
+        }
+    };
+
+    const int64_t G = (int64_t)gridDim.x * PP;
+    int64_t pen = (int64_t)blockIdx.x * PP;
+    if (pen < a.npencil) fetch(pen, t);
+    for (int i = t; i < TWN; i += NT) twl[i] = ((const cx<T>*)a.tw)[i];
+    if constexpr (!LES) {
+        for (int idx = t; idx < L * NF; idx += NT) {  // no products yet
+            const int r = idx / NF;
+            fbuf[r * LD + NI + (idx - r * NF)] = cx<T>{(T)0, (T)0};
+        }
+    }
+    int64_t prev = -1;  // DNS: group whose products sit in columns NI ..
+    for (;; pen += G) {
+        const bool have = pen < a.npencil, havep = prev >= 0;
+        if (!have && (LES || !havep)) break;
+        const int tl = opaque(t);
+        const int ti = HOISTI ? t : tl;
+        if (have) {
+            spread(ti);
+            if (pen + G < a.npencil) fetch(pen + G, ti);
+        }
+        lds_barrier();
+        auto load = [&](int b, int j, auto rc) -> cx<T> {
+            constexpr int LR0 = L / Plan<L>::r(0), p0 = LR0 * decltype(rc)::value;
+            constexpr bool IN = !LES || p0 + LR0 - 1 < NKC || p0 > L - NKC;
+            constexpr bool ZERO = LES && p0 >= NKC && p0 + LR0 - 1 <= L - NKC;
+            const int p = p0 + j;
+            if constexpr (ZERO) return cx<T>{(T)0, (T)0};
+            const cx<T> v = fbuf[p * LD + b];
+            const bool in = IN || p < NKC || p > L - NKC;
+            return cx<T>{in ? v.x : (T)0, in ? v.y : (T)0};
+        };
+        auto store = [&](int b, int p, cx<T> v) { fbuf[p * LD + b] = v; };
+        auto none = [] {};
+        FftS<T, L, NB, NT, LD, +1, true, TWM>::template run<false>(fbuf, twl, load, store, none, tl);
+        lds_barrier();
+        // -------- half spectra of the products of group gp, in columns C0 ..
+        // (DNS: those columns hold the conjugates, forward = conj(inverse(conj x)))
+        auto unpack = [&](int64_t gp, auto c0) {
+            constexpr int C0 = decltype(c0)::value;
+            constexpr T sg = LES ? (T)1 : (T)-1;
+            for (int idx = ti; idx < NF * NKC; idx += NT) {
+                const int col = idx / NKC, k = idx - col * NKC;
+                const int q = col / PP;
+                cx<T> Zk = fbuf[k * LDF + C0 + col], Zc = fbuf[(k == 0 ? 0 : L - k) * LDF + C0 + col];
+                Zk.y *= sg;
+                Zc.y *= sg;
+                const T h = (T)0.5;
+                const int64_t o = (gp + (col - q * PP)) * pitch + k;
+                typedef __attribute__((address_space(1))) cx<T>* gout;
+                const gout d0 = (gout)fld[2 * q] + o;
+                d0->x = h * (Zk.x + Zc.x);
+                d0->y = h * (Zk.y - Zc.y);
+                if (2 * q + 1 < (LES ? 9 : 3)) {
+                    const gout d1 = (gout)fld[2 * q + 1] + o;
+                    d1->x = h * (Zk.y + Zc.y);
+                    d1->y = h * (Zc.x - Zk.x);
+                }
+            }
+        };
+        if constexpr (!LES) {
+            if (havep) {
+                unpack(prev, std::integral_constant<int, NI>{});
+                lds_barrier();
+            }
+        }
+        if (have) {
+            // -------- physical space
+            constexpr int NITP = (PP * L + NT - 1) / NT;
+            cx<T> out[LES ? NITP : 1][5];  // LES: the products, until every wave has read its points
+#pragma unroll
+            for (int i = 0; i < NITP; i++) {
+                const int idx = tl + i * NT, n = idx / PP;
+                if (PP * L % NT != 0 && idx >= PP * L) continue;
+                cx<T>* row = &fbuf[n * LD + (idx - n * PP)];
+                T u, v, w, ux, uy, uz, vx, vy, vz, wx, wy, wz;
+                if constexpr (DZP) {
+                    u = row[0].x, uz = row[0].y, v = row[PP].x, vz = row[PP].y, w = row[2 * PP].x, wz = row[2 * PP].y;
+                    ux = row[3 * PP].x, uy = row[3 * PP].y, vx = row[4 * PP].x, vy = row[4 * PP].y;
+                    wx = row[5 * PP].x, wy = row[5 * PP].y;
+                } else {
+                    u = row[0].x, v = row[0].y, w = row[PP].x;
+                    ux = row[PP].y, uy = row[2 * PP].x, uz = row[2 * PP].y;
+                    vx = row[3 * PP].x, vy = row[3 * PP].y, vz = row[4 * PP].x;
+                    wx = row[4 * PP].y, wy = row[5 * PP].x, wz = row[5 * PP].y;
+                }
+                mu = fmax(mu, fabs(u));
+                mv = fmax(mv, fabs(v));
+                mw = fmax(mw, fabs(w));
+                if (sa) vmax_sa = fmax(vmax_sa, fabs((double)u) / iAx + fabs((double)v) / iAy + fabs((double)w) / iAz);  // src/HIT_LES.cpp:377
+                s2 += (double)ux * (double)ux;
+                s3 += (double)ux * (double)ux * (double)ux;
+                // advective form (src/HIT_LES.cpp:118-120)
+                const T cxv = u * ux + v * uy + w * uz;
+                const T cyv = u * vx + v * vy + w * vz;
+                const T czv = u * wx + v * wy + w * wz;
+                if constexpr (LES) {
+                    // Smagorinsky (src/HIT_LES.cpp:130-154)
+                    const T ct = (T)a.ct;
+                    T ne = (T)2.0 * ux * ux;
+                    ne += (T)2.0 * vy * vy;
+                    ne += (T)2.0 * wz * wz;
+                    ne += (uy + vx) * (uy + vx);
+                    ne += (uz + wx) * (uz + wx);
+                    ne += (vz + wy) * (vz + wy);
+                    ne = ct * sqrt(ne);
+                    out[i][0] = cx<T>{cxv, cyv};
+                    out[i][1] = cx<T>{czv, (T)(-2.0) * ne * ux};
+                    out[i][2] = cx<T>{(T)(-1.0) * ne * (uy + vx), (T)(-2.0) * ne * vy};
+                    out[i][3] = cx<T>{(T)(-1.0) * ne * (uz + wx), (T)(-1.0) * ne * (vz + wy)};
+                    out[i][4] = cx<T>{(T)(-2.0) * ne * wz, (T)0};
+                } else {
+                    row[6 * PP] = cx<T>{cxv, -cyv};
+                    row[7 * PP] = cx<T>{czv, (T)0};
+                }
+            }
+            if constexpr (LES) {
+                if constexpr (LDF != LD) lds_barrier();
+#pragma unroll
+                for (int i = 0; i < NITP; i++) {
+                    const int idx = tl + i * NT, n = idx / PP;
+                    if (PP * L % NT != 0 && idx >= PP * L) continue;
+#pragma unroll
+                    for (int q = 0; q < 5; q++) fbuf[n * LDF + q * PP + (idx - n * PP)] = out[i][q];
+                }
+                auto load_f = [&](int b, int p) -> cx<T> { return fbuf[p * LDF + b]; };
+                auto store_f = [&](int b, int p, cx<T> v) { fbuf[p * LDF + b] = v; };
+                FftS<T, L, NF, NT, LDF, -1, true, TWM>::template run<true>(fbuf, twl, load_f, store_f, none, tl);
+                lds_barrier();
+                unpack(pen, std::integral_constant<int, 0>{});
+            }
+        }
+        lds_barrier();
+        prev = have ? pen : -1;
+    }
+    z_partials<NT>(a, (double)mu, (double)mv, (double)mw, vmax_sa, s2, s3, (double*)fbuf);
+}
+
+template <typename T, int L, bool LES>
+__global__ __launch_bounds__((ZReg<T, L, LES>::NT)) __attribute__((amdgpu_waves_per_eu(ZReg<T, L, LES>::W))) void k_zreg(ZArgs a)
+{
+    zreg_body<T, L, LES>(a);
+}
+
+template <typename T, int L, bool LES>
+__global__ __launch_bounds__((ZReg<T, L, LES>::NT)) __attribute__((amdgpu_waves_per_eu(ZReg<T, L, LES>::W))) void k_zreg_b(
+    const ZArgs* __restrict__ arr, const int* __restrict__ left)
+{
+    if (left[blockIdx.y] <= 0) return;
+    zreg_body<T, L, LES>(arr[blockIdx.y]);
+}
+
+// ---------------------------------------------------------------------------
 // z pass, one wave per pencil (DNS and velocity-only modes, L = 64*E).
 // Lane t owns the physical points z = t + 64 m; the twelve fields arrive pair
 // by pair from WaveFft and the products u.grad(u) accumulate in registers in
@@ -2366,6 +2719,69 @@ hipError_t launch_strided(int L, int prec, int in_fp64, int out_fp64, int dir, c
 }
 #endif
 
+template <class K>
+static int blocks_per_cu(K kernel, int nt)
+{
+    int nb = 0;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, kernel, nt, 0) != hipSuccess) return -1;
+    return nb > 0 ? nb : 1;
+}
+
+#if SPNS_PART == 0 || SPNS_PART == 6
+template <typename T, int L, bool LES>
+static hipError_t launch_zreg_L(const ZArgs& a, int grid, hipStream_t st, const BatchLaunch* bl)
+{
+    using Z = ZReg<T, L, LES>;
+    if constexpr (LES ? Z::fits : zreg_dns<T, L>()) {
+        if (a.nk3 != Z::NKC || a.npencil % Z::PP || grid < 1) return hipErrorInvalidValue;
+        if (bl) {
+            if constexpr (batch_length(L)) {
+                hipLaunchKernelGGL((k_zreg_b<T, L, LES>), dim3((unsigned)grid, (unsigned)bl->nslots), dim3(Z::NT), 0, st,
+                                   (const ZArgs*)bl->args, bl->left);
+                return hipGetLastError();
+            }
+            return hipErrorNotSupported;
+        }
+        hipLaunchKernelGGL((k_zreg<T, L, LES>), dim3(grid), dim3(Z::NT), 0, st, a);
+        return hipGetLastError();
+    }
+    return hipErrorNotSupported;
+}
+
+hipError_t launch_zreg(int L, int prec, const ZArgs& a, int grid, hipStream_t st, const BatchLaunch* bl)
+{
+#define X(LL)                                                                                                          \
+    if (L == LL) {                                                                                                     \
+        if (prec == PREC_FP64)                                                                                         \
+            return a.les ? launch_zreg_L<double, LL, true>(a, grid, st, bl) : launch_zreg_L<double, LL, false>(a, grid, st, bl); \
+        return a.les ? launch_zreg_L<float, LL, true>(a, grid, st, bl) : launch_zreg_L<float, LL, false>(a, grid, st, bl); \
+    }
+    SPNS_FOR_EACH_L(X)
+#undef X
+    return hipErrorInvalidValue;
+}
+
+template <typename T, int L, bool LES>
+static int zreg_blocks_L()
+{
+    using Z = ZReg<T, L, LES>;
+    if constexpr (LES ? Z::fits : zreg_dns<T, L>()) return blocks_per_cu(k_zreg<T, L, LES>, Z::NT);
+    return -1;
+}
+
+int zreg_blocks(int L, int prec, bool les)
+{
+#define X(LL)                                                                                          \
+    if (L == LL) {                                                                                     \
+        if (prec == PREC_FP64) return les ? zreg_blocks_L<double, LL, true>() : zreg_blocks_L<double, LL, false>(); \
+        return les ? zreg_blocks_L<float, LL, true>() : zreg_blocks_L<float, LL, false>();             \
+    }
+    SPNS_FOR_EACH_L(X)
+#undef X
+    return -1;
+}
+#endif
+
 #if SPNS_PART == 0 || SPNS_PART == 3
 // Compile-time retained k3 count of the standard 3/2 padding (M = 3N/2,
 // nk3 = N/2 + 1 = M/3 + 1), 0 where M is not a multiple of 3.
@@ -2392,7 +2808,7 @@ static bool zstage_ok(const ZArgs& a)
 }
 
 // z-pass kernel variants and the choice among them
-enum { ZV_BLOCK, ZV_WAVE, ZV_STAGE, ZV_STAGE_NKC, ZV_FUSE_NKC };
+enum { ZV_BLOCK, ZV_WAVE, ZV_STAGE, ZV_STAGE_NKC, ZV_FUSE_NKC, ZV_REG };
 
 template <typename T, int L>
 constexpr int zfuse_nt()
@@ -2415,6 +2831,11 @@ static int zpass_pick(const ZArgs& a)
     if (a.kernel == ZK_STAGED || a.kernel == ZK_STAGED_NOFUSE) {
         const bool pitch_ok = a.pitch + zstage_pad<T>() <= zstage_spc<L>() && a.nk3 <= a.pitch;
         const bool nkc = zstage_nkc<L>() > 0 && a.nk3 == zstage_nkc<L>();
+        if constexpr (MODE == 0 && L % 3 == 0) {
+            if (a.kernel == ZK_STAGED && nkc && (a.les ? ZReg<T, L, true>::fits && a.npencil % ZReg<T, L, true>::PP == 0
+                                                       : zreg_dns<T, L>() && a.npencil % ZReg<T, L, false>::PP == 0))
+                return ZV_REG;
+        }
         if constexpr (MODE == 0 && zfuse_fits<T, L>()) {
             if (a.kernel == ZK_STAGED && !a.les && pitch_ok && nkc) return ZV_FUSE_NKC;
         }
@@ -2436,6 +2857,8 @@ static hipError_t launch_zpass_L(const ZArgs& a, int grid, hipStream_t st, const
             const dim3 g((unsigned)grid, (unsigned)bl->nslots);
             const ZArgs* arr = (const ZArgs*)bl->args;
             switch (zpass_pick<T, L, MODE>(a)) {
+            case ZV_REG:
+                return launch_zreg(L, sizeof(T) == 8 ? PREC_FP64 : PREC_FP32, a, grid, st, bl);
             case ZV_FUSE_NKC:
                 if constexpr (zfuse_fits<T, L>()) {
                     constexpr int NTF = zfuse_nt<T, L>();
@@ -2469,6 +2892,8 @@ static hipError_t launch_zpass_L(const ZArgs& a, int grid, hipStream_t st, const
             return hipGetLastError();
         }
         break;
+    case ZV_REG:
+        return launch_zreg(L, sizeof(T) == 8 ? PREC_FP64 : PREC_FP32, a, grid, st, nullptr);
     case ZV_FUSE_NKC:
         if constexpr (MODE == 0 && zfuse_fits<T, L>()) {
             constexpr int NTF = zfuse_nt<T, L>();
@@ -2501,14 +2926,6 @@ static hipError_t launch_zpass_L(const ZArgs& a, int grid, hipStream_t st, const
     }
 }
 
-template <class K>
-static int blocks_per_cu(K kernel, int nt)
-{
-    int nb = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, kernel, nt, 0) != hipSuccess) return -1;
-    return nb > 0 ? nb : 1;
-}
-
 // Grid of the z pass: the staged kernels run persistent blocks (as many as
 // fit on the device at once, counted for the full step's kernel), the others
 // one block per pencil up to 65536.
@@ -2518,7 +2935,12 @@ static int zpass_grid_L(const ZArgs& a, int64_t npen)
     constexpr int NTS = zstage_nt<T, L>();
     constexpr int NKC = zstage_nkc<L>();
     int nb = 0;
+    int64_t items = npen;
     switch (zpass_pick<T, L, 0>(a)) {
+    case ZV_REG:
+        nb = zreg_blocks(L, sizeof(T) == 8 ? PREC_FP64 : PREC_FP32, a.les);
+        items = npen / (a.les ? zreg_pp<L, true>() : zreg_pp<L, false>());
+        break;
     case ZV_FUSE_NKC:
         if constexpr (zfuse_fits<T, L>()) nb = blocks_per_cu(k_zfuse<T, L, zfuse_nt<T, L>(), NKC>, zfuse_nt<T, L>());
         break;
@@ -2537,7 +2959,7 @@ static int zpass_grid_L(const ZArgs& a, int64_t npen)
     if (hipGetDevice(&dev) != hipSuccess) return -1;
     if (hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return -1;
     const int64_t g = (int64_t)ncu * nb;
-    return (int)(npen < g ? npen : g);
+    return (int)(items < g ? items : g);
 }
 
 int zpass_grid(int L, int prec, const ZArgs& a, int64_t npen)
