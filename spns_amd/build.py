@@ -27,6 +27,7 @@ UNITS = [
     ("spns_kernels.hip", "k4.o", ["-DSPNS_PART=4"]),
     ("spns_kernels.hip", "k5.o", ["-DSPNS_PART=5"]),
     ("spns_kernels.hip", "k6.o", ["-DSPNS_PART=6"]),
+    ("spns_kernels.hip", "k7.o", ["-DSPNS_PART=7"]),
     ("spns_ctx.hip", "ctx.o", []),
     ("hit.cpp", "hit.o", []),
     ("params.cpp", "params.o", []),

@@ -290,6 +290,7 @@ static double* noalloc_scratch(int device, hipError_t* err)
 // Solver context
 // ===========================================================================
 struct spns_ctx {
+    static constexpr int kMaxPartials = 1024;  // most blocks whose shell partials the finalize sums
     spns_config cfg{};
     int Nx, Ny, Nz, Mx, My, Mz, Nx_2, Ny_2, Nz_2;
     int nk1, nk2, nk3, nbins, last_rad, last_rad_max, prec, les, rot, sa;
@@ -413,7 +414,7 @@ struct spns_ctx {
         twy = upload_twiddles(My, prec);
         twz = upload_twiddles(Mz, prec);
         alloc((void**)&scal, sizeof(DevScalars));
-        grid_epi = (int)std::min<int64_t>((nmodes_p + 255) / 256, 1024);
+        grid_epi = (int)std::min<int64_t>((nmodes_p + 255) / 256, kMaxPartials);
         const int64_t npen = (int64_t)My * Mx;
         {
             ZArgs zq{};
@@ -425,8 +426,8 @@ struct spns_ctx {
             grid_z = zpass_grid(Mz, prec, zq, npen);
             if (grid_z <= 0) throw Error(SPNS_EHIP, "z pass: no launch configuration for this length");
         }
-        alloc((void**)&hist_partial, sizeof(double) * (size_t)grid_epi * nbins);
-        alloc((void**)&om_partial, sizeof(double) * grid_epi);
+        alloc((void**)&hist_partial, sizeof(double) * (size_t)kMaxPartials * nbins);
+        alloc((void**)&om_partial, sizeof(double) * kMaxPartials);
         alloc((void**)&ed_partial, sizeof(double) * grid_epi);
         alloc((void**)&z_partial, sizeof(double) * 4 * grid_z);
         alloc((void**)&ticket, sizeof(int));
@@ -443,23 +444,21 @@ struct spns_ctx {
             HIPCHK(hipMemsetAsync(R[c], 0, tsz * (size_t)nmodes_p, st));
             if (keep_prev) HIPCHK(hipMemsetAsync(ukprev[c], 0, sb, st));
         }
-        // fused forward y pass + epilogue for DNS steps (environment
-        // SPNS_EPI=split keeps the two kernels apart)
+        // fused forward y pass + epilogue (an LES has it at short lengths only;
+        // environment SPNS_EPI=split keeps the two kernels apart)
         {
             const char* ev = std::getenv("SPNS_EPI");
             const bool split = ev && std::string(ev) == "split";
             grid_yepi = 0;
-            if (!les && !split && fwd_y_args(3).padded_ok) {
-                const int tb = strided_tile(My, prec);
-                const int64_t items = tb > 0 ? (int64_t)nk1 * ((nk3 + tb - 1) / tb) : 0;
-                if (items > 0) grid_yepi = yepi_grid(My, prec, nbins, nk2, items, grid_epi);
+            if (!split && fwd_y_args(nfwd).padded_ok) {
+                grid_yepi = yepi_grid(My, prec, nbins, nk2, nk1, nk3, kMaxPartials, false, les);
                 // the next step's inverse y pass inside the fused kernel
                 // (environment SPNS_YINV=0 keeps it a separate pass)
                 const char* yv = std::getenv("SPNS_YINV");
                 yinv = false;
                 grid_yinv = 0;
                 if (grid_yepi > 0 && !cfg.isNotCubic && !(yv && yv[0] == '0') && inv_y_args(false).padded_ok) {
-                    grid_yinv = yepi_grid(My, prec, nbins, nk2, items, grid_epi, true);
+                    grid_yinv = yepi_grid(My, prec, nbins, nk2, nk1, nk3, kMaxPartials, true, les);
                     yinv = grid_yinv > 0;
                 }
             }
@@ -731,11 +730,11 @@ struct spns_ctx {
     {
         if (yinv) {
             const StridedArgs ia = inv_y_args(false);
-            HIPCHK(launch_yepi(My, prec, fwd_y_args(3), nk1, epi_args(EPI_STEP), grid_yinv, st, nullptr, &ia, x1v));
+            HIPCHK(launch_yepi(My, prec, fwd_y_args(nfwd), nk1, epi_args(EPI_STEP), grid_yinv, st, nullptr, &ia, x1v));
             return grid_yinv;
         }
         if (grid_yepi > 0) {
-            HIPCHK(launch_yepi(My, prec, fwd_y_args(3), nk1, epi_args(EPI_STEP), grid_yepi, st));
+            HIPCHK(launch_yepi(My, prec, fwd_y_args(nfwd), nk1, epi_args(EPI_STEP), grid_yepi, st));
             return grid_yepi;
         }
         fwd_y();

@@ -195,9 +195,13 @@ hipError_t launch_line(int L, int prec, int dir, const StridedArgs& a, hipStream
 // inv: the variant with the next step's inverse y pass (k_yepi_inv), which
 // launch_yepi runs when ia (the inverse pass's arguments) is given; it sets
 // *x1v
-int yepi_grid(int L, int prec, int nbins, int nout, int64_t items, int max_grid, bool inv = false);
+int yepi_grid(int L, int prec, int nbins, int nout, int A, int B, int max_grid, bool inv, bool les);
 hipError_t launch_yepi(int L, int prec, const StridedArgs& a, int A, const EpiArgs& e, int grid, hipStream_t st,
                        const BatchLaunch* bl = nullptr, const StridedArgs* ia = nullptr, int* x1v = nullptr);
+// k_ycomb, where launch_yepi and yepi_grid pick it
+int ycomb_grid(int L, int prec, bool les, int nbins, int nout, int A, int B, int max_grid);
+hipError_t launch_ycomb(int L, int prec, const StridedArgs& a, const EpiArgs& e, int grid, hipStream_t st, const BatchLaunch* bl,
+                        const StridedArgs* ia, int* x1v);
 hipError_t launch_set_int(int* p, int v, hipStream_t st);
 hipError_t launch_epilogue(int prec, const EpiArgs& a, int grid, hipStream_t st, const BatchLaunch* bl = nullptr);
 hipError_t launch_finalize(const FinArgs& a, hipStream_t st, const BatchLaunch* bl = nullptr);

@@ -1797,23 +1797,17 @@ static __device__ __forceinline__ EpiScalars epi_scalars(const EpiArgs& a)
 // RT: the storage type of the R history (the transform type of the form:
 // the FP32-split form keeps R in FP32, whose convective part already carries
 // the FP32 transforms' rounding; R is combined in FP64 either way).
+// epi_core takes the mode's state U and history R0 already loaded.
 template <typename RT>
-static __device__ __forceinline__ void epi_mode(const EpiArgs& a, const EpiScalars& q, int64_t m, int k1, int k2, int k3,
-                                         bool step, const cx<double>* C, const cx<double>* S, double* myh, double& om,
-                                         double& ed, cx<double>* Nout = nullptr)
+static __device__ __forceinline__ void epi_core(const EpiArgs& a, const EpiScalars& q, int64_t m, int k1, int k2, int k3,
+                                         bool step, cx<double>* U, const cx<double>* R0, const cx<double>* C, const cx<double>* S,
+                                         double* myh, double& om, double& ed, cx<double>* Nout)
 {
     const int ik2 = k1 * k1 + k2 * k2 + k3 * k3;
     const double rad2 = (double)ik2;
     const int K = shell_of(ik2);
-    cx<double> U[3], R0[3], R1[3];
-#pragma unroll
-    for (int c = 0; c < 3; c++) U[c] = a.uk[c][m];
+    cx<double> R1[3];
     if (step) {
-#pragma unroll
-        for (int c = 0; c < 3; c++) {
-            const cx<RT> r = ((const cx<RT>*)a.R[c])[m];
-            R0[c] = cx<double>{(double)r.x, (double)r.y};
-        }
         const double dt = q.dt, kap = q.kap, k05 = q.k05, alpha = q.alpha;
         const double ct = q.nu * rad2;
         const bool mean = !(rad2 > 0.0);
@@ -1894,6 +1888,30 @@ static __device__ __forceinline__ void epi_mode(const EpiArgs& a, const EpiScala
     const double en = 2 * rad2 * ke;
     om += conj ? 2 * en : en;
     ed += conj ? 2 * ke : ke;
+}
+
+template <typename RT>
+static __device__ __forceinline__ void epi_load(const EpiArgs& a, int64_t m, bool step, cx<double>* U, cx<double>* R0)
+{
+#pragma unroll
+    for (int c = 0; c < 3; c++) U[c] = a.uk[c][m];
+    if (step) {
+#pragma unroll
+        for (int c = 0; c < 3; c++) {
+            const cx<RT> r = ((const cx<RT>*)a.R[c])[m];
+            R0[c] = cx<double>{(double)r.x, (double)r.y};
+        }
+    }
+}
+
+template <typename RT>
+static __device__ __forceinline__ void epi_mode(const EpiArgs& a, const EpiScalars& q, int64_t m, int k1, int k2, int k3,
+                                         bool step, const cx<double>* C, const cx<double>* S, double* myh, double& om,
+                                         double& ed, cx<double>* Nout = nullptr)
+{
+    cx<double> U[3], R0[3];
+    epi_load<RT>(a, m, step, U, R0);
+    epi_core<RT>(a, q, m, k1, k2, k3, step, U, R0, C, S, myh, om, ed, Nout);
 }
 
 // Per-wave shell histograms [NW][nbins] summed in wave order into the
@@ -2187,6 +2205,170 @@ __device__ __forceinline__ void yepi_body(const StridedArgs& a, const EpiArgs& e
         }
     }
     epi_flush<NT>(e, hist, om, (double*)fbuf);
+}
+
+// ---------------------------------------------------------------------------
+// The same at the short lengths, with an item's fields side by side: one
+// forward transform of all 3 (LES: 9) TB columns, the epilogue, and with INV one
+// inverse transform of the 6 TB columns (u_c, then d/dy u_c).  Also the LES form.
+// What bounds these sizes is the chain of transforms and barriers a block runs
+// through, not bytes: nine transforms one after the other at 48 points, two here.
+// The transform
+// buffer is the copy's target and the inverse's input, so nothing else is staged
+// and several blocks fit a CU, which hides the copies.
+// fwd_y + epilogue + next inv_y, a step: 32^3 DNS FP32 21.3 -> 5.8 us; in three
+// kernels before: 96x64x64 LES FP32 41 -> 25 us, 16 of them 616 -> 400.
+// ---------------------------------------------------------------------------
+template <typename T, int L, bool LES>
+struct YComb {
+    static constexpr int NF = LES ? 9 : 3;
+    static constexpr size_t bytes(int tb) { return sizeof(cx<T>) * L * (size_t)(NF > 6 ? NF : 6) * tb; }
+    // 4 columns at the shortest lengths: 147 against 170 us a step for 16 x 32^3
+    static constexpr int TB = L <= 48 || bytes(8) > 112 * 1024 ? 4 : 8;
+    // one butterfly a thread in every stage, as in the separate kernels: with two
+    // the compiler contracts some differently, and FP32 would not keep its bits
+    static constexpr int NT = sstage_nt<L, (NF > 6 ? NF : 6) * TB>();
+    // state and history read before the forward transform: at the shortest
+    // lengths (beyond, the registers cost more than the latency)
+    static constexpr bool PRE = L <= 72;
+    static constexpr int TWM = sizeof(T) == 8 ? 1 : 2;
+    static constexpr size_t lds = bytes(TB) + sizeof(cx<T>) * fft_twiddle_span<L, TWM>();
+    // DNS: from 96 points on the batched runs are faster with k_yepi's smaller
+    // blocks (16 x 64^3 FP32: 691 against 838 us a step; one run 97 against 84).
+    // LES, which has no other fused form: to 144 points, FP64 to 192 (128^3 870 ->
+    // 808 us; FP32 there 612 -> 606, but a batch of 16 7.80 -> 8.17 ms).
+    static constexpr bool use = L <= (!LES ? 72 : sizeof(T) == 8 ? 192 : 144) && lds <= 144 * 1024;
+};
+
+template <typename T, int L, bool LES, bool INV>
+__device__ __forceinline__ void ycomb_body(const StridedArgs& a, const EpiArgs& e, const StridedArgs& ia, int* x1v)
+{
+    using Y = YComb<T, L, LES>;
+    constexpr int TB = Y::TB, NT = Y::NT, NF = Y::NF, NW = NT / 64, TWM = Y::TWM;
+    constexpr int NBF = NF * TB, NBI = 6 * TB;
+    constexpr int TWN = fft_twiddle_span<L, TWM>();
+    constexpr int EPS = 16 / (int)sizeof(cx<T>), SPF = TB / EPS, SPR = NF * SPF;  // 16-byte copy slots per field and per row
+    constexpr int NOUTMAX = 2 * (L / 3) + 1;
+    constexpr int Q = (NOUTMAX * TB + NT - 1) / NT;
+    __shared__ __align__(16) cx<T> fbuf[L * (NBF > NBI ? NBF : NBI)];
+    __shared__ __align__(16) cx<T> twl[TWN];
+    __shared__ const cx<T>* src[NF];
+    extern __shared__ double hist[];  // [NW][nbins]
+    static_assert(sizeof(fbuf) >= NW * sizeof(double), "reduction scratch aliases fbuf");
+    const int t = threadIdx.x, nb = e.nbins;
+    if (INV && blockIdx.x == 0 && t == 0) *x1v = 1;  // read by the next step's inverse y pass only
+    if (t < NF) src[t] = (const cx<T>*)a.job[t].in;
+    for (int i = t; i < NW * nb; i += NT) hist[i] = 0.0;
+    for (int i = t; i < TWN; i += NT) twl[i] = ((const cx<T>*)a.tw)[i];
+    __syncthreads();
+    double* myh = hist + (t >> 6) * nb;
+    const EpiScalars q = epi_scalars(e);
+    double om = 0.0, ed_unused = 0.0;
+    const double inv_nf = 1.0 / e.nf;
+    const int nout = a.nout, hout = nout / 2;
+    const int ntiles = (a.B + TB - 1) / TB;
+    const int nitems = a.A * ntiles, G = gridDim.x;  // G a multiple of 8
+    const int wave = __builtin_amdgcn_readfirstlane(t >> 6), lane = t & 63;
+    const uint32_t base = lds_addr(fbuf);
+    auto none = [] {};
+    for (int it = (blockIdx.x % 8) * (G / 8) + blockIdx.x / 8; it < nitems; it += G) {
+        const int i1 = it / ntiles, b0 = (it - i1 * ntiles) * TB;
+        const int k1 = wrap_k(i1, e.nk1);
+        const int64_t off = (int64_t)i1 * a.in_a_stride + b0;
+        for (int m = wave; m * 64 < L * SPR; m += NW) {
+            const int s = m * 64 + lane;
+            const int row = s / SPR, r = s - row * SPR, f = r / SPF;
+            if (s < L * SPR) dma16(src[f] + off + (int64_t)row * a.in_row_stride + (r - f * SPF) * EPS, base + (uint32_t)m * 1024u);
+        }
+        // this thread's modes: i = k2 index, b = column
+        cx<double> U[Q][3], R0[Q][3];
+        bool ok[Q];
+#pragma unroll
+        for (int qq = 0; qq < Q; qq++) {
+            const int idx = t + qq * NT, i = idx / TB, b = idx - i * TB;
+            const int k2 = wrap_k(i, e.nk2), k3 = b0 + b;
+            ok[qq] = idx < nout * TB && k3 < a.B && !(e.notcubic && ((k1 % e.Lx) || (k2 % e.Ly) || (k3 % e.Lz)));  // src/HIT_LES.cpp:867-871
+            if (Y::PRE && ok[qq]) epi_load<T>(e, ((int64_t)i * e.nk1 + i1) * e.nk3p + k3, true, U[qq], R0[qq]);
+        }
+        dma_wait();
+        lds_barrier();
+        auto load_f = [&](int b, int p) -> cx<T> { return fbuf[p * NBF + b]; };
+        auto store_f = [&](int b, int p, cx<T> v) { fbuf[p * NBF + b] = v; };
+        FftS<T, L, NBF, NT, NBF, -1, true, TWM>::template run<false>(fbuf, twl, load_f, store_f, none, t);
+        lds_barrier();
+        cx<double> nn[Q][3];
+#pragma unroll
+        for (int qq = 0; qq < Q; qq++) {
+            const int idx = t + qq * NT, i = idx / TB, b = idx - i * TB;
+            if (ok[qq]) {
+                const int p = (i <= hout) ? i : L - (nout - i);
+                const int k2 = wrap_k(i, e.nk2), k3 = b0 + b;
+                cx<double> CS[NF];  // convective term, then SGS stress 11 21 22 31 32 33 (Fourier_Normalization)
+#pragma unroll
+                for (int f = 0; f < NF; f++) {
+                    const cx<T> v = fbuf[p * NBF + f * TB + b];
+                    CS[f] = cx<double>{(double)v.x * inv_nf, (double)v.y * inv_nf};
+                }
+                if (!Y::PRE) epi_load<T>(e, ((int64_t)i * e.nk1 + i1) * e.nk3p + k3, true, U[qq], R0[qq]);
+                epi_core<T>(e, q, ((int64_t)i * e.nk1 + i1) * e.nk3p + k3, k1, k2, k3, true, U[qq], R0[qq], CS, LES ? CS + (LES ? 3 : 0) : nullptr,
+                            myh, om, ed_unused, nn[qq]);
+            }
+        }
+        lds_barrier();  // every wave has read its transforms
+        if constexpr (INV) {
+            const int hin = ia.nin / 2;
+#pragma unroll
+            for (int qq = 0; qq < Q; qq++) {
+                const int idx = t + qq * NT, i = idx / TB, b = idx - i * TB;
+                if (ok[qq]) {
+                    const int k2 = wrap_k(i, e.nk2), p = (i <= hin) ? i : L - (ia.nin - i);
+#pragma unroll
+                    for (int c = 0; c < 3; c++) {
+                        fbuf[p * NBI + c * TB + b] = cx<T>{(T)nn[qq][c].x, (T)nn[qq][c].y};
+                        fbuf[p * NBI + (3 + c) * TB + b] = times_ik<T>((double)k2, nn[qq][c]);
+                    }
+                }
+            }
+            lds_barrier();
+            auto load_i = [&](int b, int p) -> cx<T> {
+                const cx<T> v = fbuf[p * NBI + b];
+                const bool in = p <= hin || p >= L - hin;  // else zero padding
+                return cx<T>{in ? v.x : (T)0, in ? v.y : (T)0};
+            };
+            auto store_i = [&](int b, int p, cx<T> v) { fbuf[p * NBI + b] = v; };
+            FftS<T, L, NBI, NT, NBI, +1, true, TWM>::template run<false>(fbuf, twl, load_i, store_i, none, t);
+            lds_barrier();
+#pragma unroll
+            for (int c = 0; c < 6; c++) {
+                cx<T>* o = (cx<T>*)(c < 3 ? ia.job[c % 3].out : ia.job[c % 3].out2) + (int64_t)i1 * ia.out_a_stride + b0;
+                for (int idx = t; idx < L * TB; idx += NT) {
+                    const int i = idx / TB, b = idx - i * TB;
+                    if (b0 + b < ia.B) o[(int64_t)i * ia.out_row_stride + b] = fbuf[i * NBI + c * TB + b];
+                }
+            }
+            lds_barrier();
+        }
+    }
+    epi_flush<NT>(e, hist, om, (double*)fbuf);
+}
+
+template <typename T, int L, bool LES, bool INV>
+__global__ __launch_bounds__((YComb<T, L, LES>::NT)) void k_ycomb(StridedArgs a, EpiArgs e, StridedArgs ia, int* x1v)
+{
+    ycomb_body<T, L, LES, INV>(a, e, ia, x1v);
+}
+
+template <typename T, int L, bool LES, bool INV>
+__global__ __launch_bounds__((YComb<T, L, LES>::NT)) void k_ycomb_b(const StridedArgs* __restrict__ arr, const EpiArgs* __restrict__ earr,
+                                                                    const StridedArgs* __restrict__ iarr, const int* __restrict__ left)
+{
+    if (left[blockIdx.y] <= 0) return;
+    if constexpr (INV) {
+        const StridedArgs& ia = iarr[blockIdx.y];
+        ycomb_body<T, L, LES, true>(arr[blockIdx.y], earr[blockIdx.y], ia, ia.setflag);
+    } else {
+        ycomb_body<T, L, LES, false>(arr[blockIdx.y], earr[blockIdx.y], arr[blockIdx.y], nullptr);
+    }
 }
 
 template <typename T, int L, int TB, int NT>
@@ -2782,6 +2964,100 @@ int zreg_blocks(int L, int prec, bool les)
 }
 #endif
 
+#if SPNS_PART == 0 || SPNS_PART == 7
+// Grid of k_ycomb: both forms (with and without the inverse pass) take the
+// smaller of their occupancies, so that the shell partials are the same.
+template <typename T, int L, bool LES>
+static int ycomb_grid_L(int nbins, int nout, int A, int B, int max_grid)
+{
+    using Y = YComb<T, L, LES>;
+    if (nout > 2 * (L / 3) + 1) return 0;
+    const size_t shm = sizeof(double) * (Y::NT / 64) * (size_t)nbins;
+    if (Y::lds + shm + 256 > 160 * 1024 - 512) return 0;
+    int n0 = 0, n1 = 0, dev = 0, ncu = 0;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n0, k_ycomb<T, L, LES, false>, Y::NT, shm) != hipSuccess || n0 < 1) return 0;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n1, k_ycomb<T, L, LES, true>, Y::NT, shm) != hipSuccess || n1 < 1) return 0;
+    if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return 0;
+    int64_t g = (int64_t)ncu * (n0 < n1 ? n0 : n1);
+    const int64_t items = (int64_t)A * ((B + Y::TB - 1) / Y::TB);
+    if (items < g) g = items;
+    g = (g + 7) / 8 * 8;
+    return (int)(g > max_grid ? max_grid / 8 * 8 : g);
+}
+
+template <typename T, int L, bool LES>
+static hipError_t launch_ycomb_L(const StridedArgs& a, const EpiArgs& e, int grid, hipStream_t st, const BatchLaunch* bl, const StridedArgs* ia,
+                                 int* x1v)
+{
+    using Y = YComb<T, L, LES>;
+    const size_t shm = sizeof(double) * (Y::NT / 64) * (size_t)e.nbins;
+    if (bl) {
+        if constexpr (batch_length(L)) {
+            const dim3 g(grid, bl->nslots);
+            if (ia)
+                hipLaunchKernelGGL((k_ycomb_b<T, L, LES, true>), g, dim3(Y::NT), shm, st, (const StridedArgs*)bl->args, (const EpiArgs*)bl->args2,
+                                   (const StridedArgs*)bl->args3, bl->left);
+            else
+                hipLaunchKernelGGL((k_ycomb_b<T, L, LES, false>), g, dim3(Y::NT), shm, st, (const StridedArgs*)bl->args, (const EpiArgs*)bl->args2,
+                                   (const StridedArgs*)bl->args3, bl->left);
+            return hipGetLastError();
+        }
+        return hipErrorNotSupported;
+    }
+    if (ia) hipLaunchKernelGGL((k_ycomb<T, L, LES, true>), dim3(grid), dim3(Y::NT), shm, st, a, e, *ia, x1v);
+    else hipLaunchKernelGGL((k_ycomb<T, L, LES, false>), dim3(grid), dim3(Y::NT), shm, st, a, e, a, nullptr);
+    return hipGetLastError();
+}
+
+// the length's k_ycomb, where it is used (ycomb_use): f(L, T, LES) below
+#define SPNS_YCOMB_CALL(FN, ...)                                                                              \
+    if constexpr (YComb<T, LL_, true>::use) {                                                                 \
+        if (les) return FN<T, LL_, true>(__VA_ARGS__);                                                        \
+    }                                                                                                         \
+    if constexpr (YComb<T, LL_, false>::use) {                                                                \
+        if (!les) return FN<T, LL_, false>(__VA_ARGS__);                                                      \
+    }
+
+template <typename T, int LL_>
+static int ycomb_grid_any(bool les, int nbins, int nout, int A, int B, int max_grid)
+{
+    SPNS_YCOMB_CALL(ycomb_grid_L, nbins, nout, A, B, max_grid)
+    return 0;
+}
+
+template <typename T, int LL_>
+static hipError_t launch_ycomb_any(bool les, const StridedArgs& a, const EpiArgs& e, int grid, hipStream_t st, const BatchLaunch* bl,
+                                   const StridedArgs* ia, int* x1v)
+{
+    SPNS_YCOMB_CALL(launch_ycomb_L, a, e, grid, st, bl, ia, x1v)
+    return hipErrorNotSupported;
+}
+#undef SPNS_YCOMB_CALL
+
+int ycomb_grid(int L, int prec, bool les, int nbins, int nout, int A, int B, int max_grid)
+{
+#define X(LL)                                                                                              \
+    if (L == LL)                                                                                           \
+        return prec == PREC_FP64 ? ycomb_grid_any<double, LL>(les, nbins, nout, A, B, max_grid)            \
+                                 : ycomb_grid_any<float, LL>(les, nbins, nout, A, B, max_grid);
+    SPNS_FOR_EACH_L(X)
+#undef X
+    return 0;
+}
+
+hipError_t launch_ycomb(int L, int prec, const StridedArgs& a, const EpiArgs& e, int grid, hipStream_t st, const BatchLaunch* bl,
+                        const StridedArgs* ia, int* x1v)
+{
+#define X(LL)                                                                                              \
+    if (L == LL)                                                                                           \
+        return prec == PREC_FP64 ? launch_ycomb_any<double, LL>(e.les, a, e, grid, st, bl, ia, x1v)        \
+                                 : launch_ycomb_any<float, LL>(e.les, a, e, grid, st, bl, ia, x1v);
+    SPNS_FOR_EACH_L(X)
+#undef X
+    return hipErrorInvalidValue;
+}
+#endif
+
 #if SPNS_PART == 0 || SPNS_PART == 3
 // Compile-time retained k3 count of the standard 3/2 padding (M = 3N/2,
 // nk3 = N/2 + 1 = M/3 + 1), 0 where M is not a multiple of 3.
@@ -3192,13 +3468,18 @@ static int yepi_blocks_per_cu(K kern, int nbins, int max_spill)
 }
 
 template <typename T, int L>
-static int yepi_grid_L(int nbins, int nout, int64_t items, int max_grid, bool inv)
+static int yepi_grid_L(int nbins, int nout, int A, int B, int max_grid, bool inv, bool les)
 {
+    if (les ? YComb<T, L, true>::use : YComb<T, L, false>::use)
+        return ycomb_grid(L, sizeof(T) == 8 ? PREC_FP64 : PREC_FP32, les, nbins, nout, A, B, max_grid);
+    if (les) return 0;
+
     constexpr int TB = strided_tb<T, L>();
     if constexpr (TB <= 0 || (TB * sizeof(cx<T>)) % 16 != 0) {
         return 0;
     } else {
         if (nout > 2 * (L / 3) + 1) return 0;
+        const int64_t items = (int64_t)A * ((B + TB - 1) / TB);
         constexpr int NT = yepi_nt<L, TB>();
         // a variant that spills registers (the 1024-thread tiles) is slower
         // than the two separate kernels; k_yepi_inv may keep a few
@@ -3218,12 +3499,12 @@ static int yepi_grid_L(int nbins, int nout, int64_t items, int max_grid, bool in
     }
 }
 
-int yepi_grid(int L, int prec, int nbins, int nout, int64_t items, int max_grid, bool inv)
+int yepi_grid(int L, int prec, int nbins, int nout, int A, int B, int max_grid, bool inv, bool les)
 {
 #define X(LL)                                                                                   \
     if (L == LL)                                                                                \
-        return prec == PREC_FP64 ? yepi_grid_L<double, LL>(nbins, nout, items, max_grid, inv) \
-                                 : yepi_grid_L<float, LL>(nbins, nout, items, max_grid, inv);
+        return prec == PREC_FP64 ? yepi_grid_L<double, LL>(nbins, nout, A, B, max_grid, inv, les) \
+                                 : yepi_grid_L<float, LL>(nbins, nout, A, B, max_grid, inv, les);
     SPNS_FOR_EACH_L(X)
 #undef X
     return 0;
@@ -3239,7 +3520,22 @@ static hipError_t launch_yepi_L(const StridedArgs& a, int A, const EpiArgs& e, i
     } else {
         StridedArgs b = a;
         b.A = A;
-        if (!a.padded_ok || a.nin != L || a.njobs != 3 || a.nout > 2 * (L / 3) + 1 || grid < 8 || grid % 8) return hipErrorInvalidValue;
+        if (!a.padded_ok || a.nin != L || a.njobs != (e.les ? 9 : 3) || a.nout > 2 * (L / 3) + 1 || grid < 8 || grid % 8)
+            return hipErrorInvalidValue;
+        if (e.les ? YComb<T, L, true>::use : YComb<T, L, false>::use) {
+            StridedArgs ib{};
+            if (ia) {
+                // the inverse pass's items must be the forward pass's
+                bool ok = (bl ? bl->args3 && ia->setflag : x1v != nullptr) && ia->padded_ok && ia->njobs == 3 && ia->nout == L &&
+                          ia->nin == a.nout && ia->B == a.B;
+                for (int j = 0; ok && j < 3; j++) ok = ia->job[j].in && ia->job[j].out && ia->job[j].out2;
+                if (!ok) return hipErrorInvalidValue;
+                ib = *ia;
+                ib.A = A;
+            }
+            return launch_ycomb(L, sizeof(T) == 8 ? PREC_FP64 : PREC_FP32, b, e, grid, st, bl, ia ? &ib : nullptr, x1v);
+        }
+        if (e.les) return hipErrorNotSupported;
         if (bl) {
             constexpr int NT = yepi_nt<L, TB>();
             const size_t shm = sizeof(double) * (NT / 64) * (size_t)e.nbins;
