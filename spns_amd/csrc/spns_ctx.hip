@@ -333,8 +333,12 @@ struct spns_ctx {
     int grid_epi = 0, grid_z = 0;
     int grid_yepi = 0;  // > 0: the DNS step fuses its forward y pass with the epilogue (k_yepi)
     int zkernel = ZK_STAGED;  // z-pass kernel (environment SPNS_ZPASS=staged|nofuse|block|wave overrides)
-    hipGraphExec_t graph = nullptr;
-    bool graph_ready = false;
+    // captured steps: [0] whole, [1] without the inverse y pass, for a step that
+    // follows one of this context's own that left X1 current (x1_cur: x1v as
+    // the host knows it; a batch's steps set x1v alone, and [0] then skips it
+    // on the device)
+    hipGraphExec_t graph[2] = {};
+    bool x1_cur = false;
     HostCopy hcopy;
     std::string err;
     double last_ms = 0.0;
@@ -495,11 +499,10 @@ struct spns_ctx {
         ct = cfg.C_Smag * cfg.C_Smag * delta * delta;  // src/HIT_LES.cpp:132
         rot = (std::fabs(cfg.omega_x) > 0 || std::fabs(cfg.omega_y) > 0 || std::fabs(cfg.omega_z) > 0);
         (void)old;
-        if (graph) {
-            hipGraphExecDestroy(graph);
-            graph = nullptr;
+        for (hipGraphExec_t& g : graph) {
+            if (g) hipGraphExecDestroy(g);
+            g = nullptr;
         }
-        graph_ready = false;
         const size_t sb = sizeof(cx<double>) * (size_t)nmodes_p;
         for (int c3 = 0; c3 < 3; c3++) {
             HIPCHK(hipMemsetAsync(uk[c3], 0, sb, st));
@@ -525,7 +528,8 @@ struct spns_ctx {
     void release()
     {
         hcopy.release();
-        if (graph) hipGraphExecDestroy(graph);
+        for (hipGraphExec_t g : graph)
+            if (g) hipGraphExecDestroy(g);
         for (int c = 0; c < 3; c++) { hipFree(uk[c]); hipFree(R[c]); hipFree(ukprev[c]); }
         hipFree(X1); hipFree(X2); hipFree(twx); hipFree(twy); hipFree(twz);
         hipFree(scal); hipFree(hist_partial); hipFree(om_partial); hipFree(ed_partial); hipFree(z_partial); hipFree(ticket);
@@ -573,6 +577,7 @@ struct spns_ctx {
     // changed, or X1 was rewritten outside a step)
     void x1_stale()
     {
+        x1_cur = false;
         if (yinv) HIPCHK(launch_set_int(x1v, 0, st));
     }
 
@@ -785,9 +790,10 @@ struct spns_ctx {
         return f;
     }
 
-    void enqueue_step()
+    // x1: X1 holds this state's inverse y pass already
+    void enqueue_step(bool x1)
     {
-        inv_y(false);
+        if (!x1) inv_y(false);
         inv_x(false);
         zpass(0);
         fwd_x();
@@ -850,25 +856,30 @@ struct spns_ctx {
     void step(int n)
     {
         HIPCHK(hipEventRecord(ev0, st));
-        if (cfg.use_graph) {
-            if (!graph_ready) {
-                hipGraph_t g;
-                HIPCHK(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
-                try {
-                    enqueue_step();
-                } catch (...) {
-                    hipGraph_t dummy;
-                    hipStreamEndCapture(st, &dummy);
-                    throw;
+        for (int i = 0; i < n; i++) {
+            const bool x1 = yinv && x1_cur;
+            if (cfg.use_graph) {
+                hipGraphExec_t& ge = graph[x1];
+                if (!ge) {
+                    hipGraph_t g;
+                    HIPCHK(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
+                    try {
+                        enqueue_step(x1);
+                    } catch (...) {
+                        hipGraph_t dummy;
+                        hipStreamEndCapture(st, &dummy);
+                        throw;
+                    }
+                    HIPCHK(hipStreamEndCapture(st, &g));
+                    const hipError_t e = hipGraphInstantiate(&ge, g, nullptr, nullptr, 0);
+                    hipGraphDestroy(g);
+                    HIPCHK(e);
                 }
-                HIPCHK(hipStreamEndCapture(st, &g));
-                HIPCHK(hipGraphInstantiate(&graph, g, nullptr, nullptr, 0));
-                HIPCHK(hipGraphDestroy(g));
-                graph_ready = true;
+                HIPCHK(hipGraphLaunch(ge, st));
+            } else {
+                enqueue_step(x1);
             }
-            for (int i = 0; i < n; i++) HIPCHK(hipGraphLaunch(graph, st));
-        } else {
-            for (int i = 0; i < n; i++) enqueue_step();
+            x1_cur = yinv;  // the fused kernel has set x1v
         }
         HIPCHK(hipEventRecord(ev1, st));
     }
@@ -1128,14 +1139,18 @@ struct spns_batch {
 
     // one step of every live slot: the single-run step's launches
     // (spns_ctx::enqueue_step), each once over all slots
-    void enqueue_step()
+    // first: the chunk's first step, the only one whose X1 may be stale (a slot
+    // that steps has run the fused kernel in the step before)
+    void enqueue_step(bool first)
     {
         spns_ctx* c = rep;
         const int p = c->prec;
         auto bl = [&](const void* a, const void* a2 = nullptr) { return BatchLaunch{a, a2, d_left, nslots}; };
         BatchLaunch b;
-        b = bl(d_invy);
-        HIPCHK(launch_strided(c->My, p, 1, p == PREC_FP64, +1, hs[slot_of(c)].invy, c->nk1, st, &b));
+        if (first || !c->yinv) {
+            b = bl(d_invy);
+            HIPCHK(launch_strided(c->My, p, 1, p == PREC_FP64, +1, hs[slot_of(c)].invy, c->nk1, st, &b));
+        }
         b = bl(d_invx);
         HIPCHK(launch_strided(c->Mx, p, p == PREC_FP64, p == PREC_FP64, +1, hs[slot_of(c)].invx, c->My, st, &b));
         b = bl(d_z);
@@ -1183,7 +1198,7 @@ struct spns_batch {
             hipGraph_t g;
             HIPCHK(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
             try {
-                for (int i = 0; i < chunk; i++) enqueue_step();
+                for (int i = 0; i < chunk; i++) enqueue_step(i == 0);
             } catch (...) {
                 hipGraph_t dummy;
                 hipStreamEndCapture(st, &dummy);

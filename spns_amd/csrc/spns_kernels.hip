@@ -345,20 +345,50 @@ __global__ __launch_bounds__(NT) void k_sstage_b(const StridedArgs* __restrict__
 // ---------------------------------------------------------------------------
 // Block reductions
 // ---------------------------------------------------------------------------
-// Fixed-order sums and maxima: within a wave by shuffles (lane i with lane
-// i + 32, 16, ... 1), then over the waves in order through LDS.
-__device__ __forceinline__ double wave_sum(double v)
+// Fixed-order sums and maxima: within a wave by DPP moves, then over the waves
+// in order through LDS.  (A shuffle goes through LDS: six dependent ones cost
+// about 1200 cycles, these about 100.)
+// v of the lane DPP control CTRL names, 0 where there is none or its row is not
+// in RMASK
+template <int CTRL, int RMASK>
+__device__ __forceinline__ double dpp_from(double v)
 {
-#pragma unroll
-    for (int s = 32; s > 0; s >>= 1) v = v + __shfl_down(v, s);
-    return v;
+    const long long b = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_update_dpp(0, (int)b, CTRL, RMASK, 0xf, true);
+    const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, RMASK, 0xf, true);
+    return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
 }
 
-__device__ __forceinline__ double wave_max(double v)
+__device__ __forceinline__ double lane_value(double v, int lane)  // lane: uniform
 {
-#pragma unroll
-    for (int s = 32; s > 0; s >>= 1) v = fmax(v, __shfl_down(v, s));
-    return v;
+    const long long b = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_readlane((int)b, lane), hi = __builtin_amdgcn_readlane((int)(b >> 32), lane);
+    return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
+}
+
+// Over the wave's 64 lanes (all active): prefixes within each row of 16 (row
+// shifts by 1, 2, 4, 8), then row ends into the next rows (broadcasts of lanes
+// 15 and 31); lane 63 holds the whole, which every lane returns.
+__device__ __forceinline__ double wave_sum(double v)
+{
+    v = v + dpp_from<0x111, 0xf>(v);
+    v = v + dpp_from<0x112, 0xf>(v);
+    v = v + dpp_from<0x114, 0xf>(v);
+    v = v + dpp_from<0x118, 0xf>(v);
+    v = v + dpp_from<0x142, 0xa>(v);
+    v = v + dpp_from<0x143, 0xc>(v);
+    return lane_value(v, 63);
+}
+
+__device__ __forceinline__ double wave_max(double v)  // v >= 0
+{
+    v = fmax(v, dpp_from<0x111, 0xf>(v));
+    v = fmax(v, dpp_from<0x112, 0xf>(v));
+    v = fmax(v, dpp_from<0x114, 0xf>(v));
+    v = fmax(v, dpp_from<0x118, 0xf>(v));
+    v = fmax(v, dpp_from<0x142, 0xa>(v));
+    v = fmax(v, dpp_from<0x143, 0xc>(v));
+    return lane_value(v, 63);
 }
 
 // Sum over the block, in every thread; sh: NT / 64 doubles (free again on return).
@@ -371,9 +401,37 @@ __device__ __forceinline__ double block_sum(double v, double* sh)
     if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = v;
     __syncthreads();
     double r = sh[0];
+#pragma unroll
     for (int w = 1; w < NW; w++) r = r + sh[w];
     __syncthreads();
     return r;
+}
+
+// NV block-wide values at once (the first NS are sums, the rest maxima of
+// values >= 0), for the threads of wave 0; sh: NV NT / 64 doubles.
+template <int NT, int NV, int NS>
+__device__ __forceinline__ void block_reduce(double* v, double* sh)
+{
+    constexpr int NW = NT / 64;
+#pragma unroll
+    for (int i = 0; i < NV; i++) v[i] = i < NS ? wave_sum(v[i]) : wave_max(v[i]);
+    __syncthreads();
+    if ((threadIdx.x & 63) == 0) {
+#pragma unroll
+        for (int i = 0; i < NV; i++) sh[NV * (threadIdx.x >> 6) + i] = v[i];
+    }
+    __syncthreads();
+    if (threadIdx.x < 64) {  // lane i takes value i over the waves
+        const int i = threadIdx.x < NV ? threadIdx.x : 0;
+        double r = sh[i];
+#pragma unroll
+        for (int w = 1; w < NW; w++) {
+            const double x = sh[NV * w + i];
+            r = i < NS ? r + x : fmax(r, x);
+        }
+#pragma unroll
+        for (int k = 0; k < NV; k++) v[k] = lane_value(r, k);
+    }
 }
 
 // The z pass's block partials, [4] per block: sums s2, s3; the block's CFL
@@ -385,27 +443,14 @@ __device__ __forceinline__ double block_sum(double v, double* sh)
 template <int NT>
 __device__ __forceinline__ void z_partials(const ZArgs& a, double mu, double mv, double mw, double vsa, double s2, double s3, double* sh)
 {
-    constexpr int NW = NT / 64;
-    const double r[6] = {wave_max(mu), wave_max(mv), wave_max(mw), wave_max(vsa), wave_sum(s2), wave_sum(s3)};
-    __syncthreads();
-    if ((threadIdx.x & 63) == 0) {
-#pragma unroll
-        for (int i = 0; i < 6; i++) sh[6 * (threadIdx.x >> 6) + i] = r[i];
-    }
-    __syncthreads();
+    double q[6] = {s2, s3, mu, mv, mw, vsa};
+    block_reduce<NT, 6, 2>(q, sh);
     if (threadIdx.x == 0) {
-        double q[6];
-#pragma unroll
-        for (int i = 0; i < 6; i++) q[i] = sh[i];
-        for (int w = 1; w < NW; w++) {
-#pragma unroll
-            for (int i = 0; i < 6; i++) q[i] = i < 4 ? fmax(q[i], sh[6 * w + i]) : q[i] + sh[6 * w + i];
-        }
         double* o = a.z_partial + 4 * (int64_t)blockIdx.x;
-        o[0] = q[4];
-        o[1] = q[5];
-        o[2] = fmax(q[0] / a.Ax, fmax(q[1] / a.Ay, q[2] / a.Az));
-        o[3] = q[3];
+        o[0] = q[0];
+        o[1] = q[1];
+        o[2] = fmax(q[2] / a.Ax, fmax(q[3] / a.Ay, q[4] / a.Az));
+        o[3] = q[5];
     }
 }
 
@@ -2416,110 +2461,115 @@ static __device__ double FuG(double x, double a, double b, double c, double x0, 
 // Finalize: fixed-order sums of the partials; time step (src/HIT_LES.cpp:365-403)
 // With FIN_REDUCE the grid has one block per 64 shells: block x sums its
 // shells' block partials (wave w takes rows w, w + 16, ...), and the block that
-// arrives last does the rest.  What bounds it is the latency of dependent reads
-// of partials that other XCDs wrote, so rows are read eight at a time.  One
-// block over all shells took 60 us at 512^3 DNS (256 x 445 partials) and 51 at
-// 256^3 LES (1024 x 223); this 20 and 26.
+// arrives last does the rest.  What bounds it is latency: of the partials'
+// reads, which other XCDs wrote (so a shell's rows are read sixteen at a time
+// and every read that depends on nothing is issued first), and of the exchanges
+// between the waves (one for all block sums; the shells go from block to block
+// through one wave's fence and reads).  One block that summed part after part
+// took 60 us at 512^3 DNS (256 x 445 partials), 51 at 256^3 LES (1024 x 223) and
+// 10.4 at 32^3; this 9, 17 and 5.8.
 // Returns whether this block was the last one of its context's launch.
 // ---------------------------------------------------------------------------
 template <int NT>
 __device__ __forceinline__ bool finalize_body(const FinArgs& a)
 {
-    constexpr int NW = NT / 64;
-    __shared__ double red[NW];
+    constexpr int NW = NT / 64, U = 16, UZ = 3;
+    __shared__ double q[NW][64];
+    __shared__ double red[NW * 6];
+    __shared__ int last;
     DevScalars* s = a.scal;
-    const int t = threadIdx.x;
-    if (a.flags & FIN_REDUCE) {
-        __shared__ double q[NW][64];
-        __shared__ int last;
-        const int lane = t & 63, w = t >> 6;
-        const int K = blockIdx.x * 64 + lane;
-        constexpr int U = 8;
-        double acc[U] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
-        if (K < a.nbins) {
-            int b = w;
-            for (; b + (U - 1) * NW < a.nblk_epi; b += U * NW) {
+    const int t = threadIdx.x, lane = t & 63, w = t >> 6;
+    const bool zsum = a.flags & (FIN_SKEW | FIN_EPHYS | FIN_MAXVEL);
+    const int K = blockIdx.x * 64 + lane;
+    const double nu = s->nu;
+    double om = 0.0, ed = 0.0, s2 = 0.0, s3 = 0.0, mx = 0.0, mxs = 0.0;
+    double z[UZ][4];
 #pragma unroll
-                for (int u = 0; u < U; u++) acc[u] += a.hist_partial[(int64_t)(b + u * NW) * a.nbins + K];
-            }
-            for (; b < a.nblk_epi; b += NW) acc[0] += a.hist_partial[(int64_t)b * a.nbins + K];
+    for (int u = 0; u < UZ; u++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) z[u][i] = (zsum && t + u * NT < a.nblk_z) ? a.z_partial[4 * (t + u * NT) + i] : 0.0;
+    if ((a.flags & FIN_REDUCE) && t < a.nblk_epi) om = a.om_partial[t];
+    if ((a.flags & FIN_EFOUR) && t < a.nblk_epi) ed = a.ed_partial[t];
+    double e = 0.0, ef = 0.0;  // wave 0: its lanes' shells
+    if (a.flags & FIN_REDUCE) {
+        double acc = 0.0;
+        for (int b = w; b < a.nblk_epi; b += U * NW) {
+            double h[U];
+#pragma unroll
+            for (int u = 0; u < U; u++)
+                h[u] = (K < a.nbins && b + u * NW < a.nblk_epi) ? a.hist_partial[(int64_t)(b + u * NW) * a.nbins + K] : 0.0;
+#pragma unroll
+            for (int d = U / 2; d > 0; d >>= 1)
+#pragma unroll
+                for (int u = 0; u < d; u++) h[u] += h[u + d];
+            acc += h[0];
         }
-        q[w][lane] = ((acc[0] + acc[1]) + (acc[2] + acc[3])) + ((acc[4] + acc[5]) + (acc[6] + acc[7]));
+        q[w][lane] = acc;
         __syncthreads();
-        if (w == 0 && K < a.nbins) {
-            double e = q[0][lane];
-            for (int i = 1; i < NW; i++) e += q[i][lane];
-            a.ek[K] = e;
+        if (w == 0) {
+            if (K < a.nbins) {
+                e = q[0][lane];
+#pragma unroll
+                for (int i = 1; i < NW; i++) e += q[i][lane];
+                a.ek[K] = e;
+            }
+            if (gridDim.x > 1) {
+                // this block's shells (all written by this wave) before its
+                // count; the last block leaves the counter at 0
+                __threadfence();
+                if (lane == 0) {
+                    last = atomicAdd(a.ticket, 1) == (int)gridDim.x - 1;
+                    if (last) atomicExch(a.ticket, 0);
+                }
+                __threadfence();
+            }
         }
         if (gridDim.x > 1) {
-            // publish this block's shells, then count it in; the last block
-            // sees every shell and leaves the counter at 0 for the next launch
-            __threadfence();
-            __syncthreads();
-            if (t == 0) {
-                last = atomicAdd(a.ticket, 1) == (int)gridDim.x - 1;
-                if (last) atomicExch(a.ticket, 0);
-            }
             __syncthreads();
             if (!last) return false;
-            __threadfence();
-        } else {
-            __syncthreads();
+            if (w == 0) {
+                e = 0.0;
+                for (int k = lane; k < a.nbins; k += 64) {
+                    const double v = a.ek[k];
+                    e += v;
+                    if (k >= a.kfmin && k <= a.kfmax) ef += v;
+                }
+            }
+        } else if (w == 0 && K >= a.kfmin && K <= a.kfmax) {
+            ef = e;
         }
-        double om = 0.0, e = 0.0, ef = 0.0;
-        for (int b = t; b < a.nblk_epi; b += NT) om += a.om_partial[b];
-        for (int k = t; k < a.nbins; k += NT) {
-            const double v = a.ek[k];
-            e += v;
-            if (k >= a.kfmin && k <= a.kfmax) ef += v;
+        for (int b = t + NT; b < a.nblk_epi; b += NT) om += a.om_partial[b];
+    }
+    if (a.flags & FIN_EFOUR)
+        for (int b = t + NT; b < a.nblk_epi; b += NT) ed += a.ed_partial[b];
+#pragma unroll
+    for (int u = 0; u < UZ; u++) { s2 += z[u][0]; s3 += z[u][1]; mx = fmax(mx, z[u][2]); mxs = fmax(mxs, z[u][3]); }
+    if (zsum)
+        for (int b = t + UZ * NT; b < a.nblk_z; b += NT) {
+            s2 += a.z_partial[4 * b];
+            s3 += a.z_partial[4 * b + 1];
+            mx = fmax(mx, a.z_partial[4 * b + 2]);
+            mxs = fmax(mxs, a.z_partial[4 * b + 3]);
         }
-        om = block_sum<NT>(om, red);
-        e = block_sum<NT>(e, red);
-        ef = block_sum<NT>(ef, red);
-        if (t == 0) {
+    if (w == 0) {
+        e = wave_sum(e);
+        ef = wave_sum(ef);
+    }
+    double v[6] = {om, ed, s2, s3, mx, mxs};
+    block_reduce<NT, 6, 4>(v, red);
+    if (t == 0) {
+        if (a.flags & FIN_REDUCE) {
             s->ek = e;
-            s->om = om;
-            s->relambda = e / s->nu * sqrt(20.0 / 3.0 / om);
+            s->om = v[0];
+            s->relambda = e / nu * sqrt(20.0 / 3.0 / v[0]);
             // constant-power coefficient for the next step (src/HIT_LES.cpp:251-256)
             s->alpha = (ef > 1e-30) ? a.force_eps / (2.0 * ef) : 0.0;
         }
-    }
-    if (a.flags & FIN_SKEW) {
-        double s2 = 0.0, s3 = 0.0;
-        for (int b = t; b < a.nblk_z; b += NT) { s2 += a.z_partial[4 * b]; s3 += a.z_partial[4 * b + 1]; }
-        s2 = block_sum<NT>(s2, red);
-        s3 = block_sum<NT>(s3, red);
-        if (t == 0) { s->skew2 = s2; s->skew3 = s3; }
-    }
-    if (a.flags & FIN_EFOUR) {
-        double e = 0.0;
-        for (int b = t; b < a.nblk_epi; b += NT) e += a.ed_partial[b];
-        e = block_sum<NT>(e, red);
-        if (t == 0) s->ek_four = e;
-    }
-    if (a.flags & FIN_EPHYS) {
-        double e = 0.0;
-        for (int b = t; b < a.nblk_z; b += NT) e += a.z_partial[4 * b];
-        e = block_sum<NT>(e, red);
-        if (t == 0) s->ek_phys = e;
-    }
-    if (a.flags & FIN_MAXVEL) {
-        double v = 0.0, vs = 0.0;
-        for (int b = t; b < a.nblk_z; b += NT) { v = fmax(v, a.z_partial[4 * b + 2]); vs = fmax(vs, a.z_partial[4 * b + 3]); }
-        v = wave_max(v);
-        vs = wave_max(vs);
-        __shared__ double mx[NW][2];
-        if ((t & 63) == 0) { mx[t >> 6][0] = v; mx[t >> 6][1] = vs; }
-        __syncthreads();
-        if (t == 0) {
-            for (int w = 1; w < NW; w++) { v = fmax(v, mx[w][0]); vs = fmax(vs, mx[w][1]); }
-            s->maxvel = v;
-            s->maxvel_sa = vs;
-        }
-    }
-    if (t == 0) {
+        if (a.flags & FIN_SKEW) { s->skew2 = v[2]; s->skew3 = v[3]; }
+        if (a.flags & FIN_EFOUR) s->ek_four = v[1];
+        if (a.flags & FIN_EPHYS) s->ek_phys = v[2];
+        if (a.flags & FIN_MAXVEL) { s->maxvel = v[4]; s->maxvel_sa = v[5]; }
         if (a.flags & FIN_DT) {
-            const double nu = s->nu;
             if (a.sa) {
                 const double MaxVel = s->maxvel_sa, Ah = a.Ah;
                 const double phi0 = atan(MaxVel * Ah * Ah / (0.35 * nu * 12.0));
