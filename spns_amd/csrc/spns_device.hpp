@@ -369,18 +369,6 @@ __device__ __forceinline__ void dma16(const void* g, uint32_t lds_base)
         : "memory");
 }
 
-// The same for 4 bytes per lane (active lane i's bytes land at lds_base + 4*i),
-// for rows that are only 4- or 8-byte aligned.
-__device__ __forceinline__ void dma4(const void* g, uint32_t lds_base)
-{
-    uint32_t saved;
-    asm volatile(
-        "s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %2, off\n\ts_mov_b32 m0, %0"
-        : "=&s"(saved)
-        : "s"(lds_base), "v"(g)
-        : "memory");
-}
-
 // An opaque copy of v: the compiler cannot see through it, so values derived
 // from it are not hoisted out of the enclosing loop.
 __device__ __forceinline__ int opaque(int v)

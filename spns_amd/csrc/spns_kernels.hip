@@ -59,6 +59,14 @@ __device__ __forceinline__ cx<T> times_ik(TIN kk, cx<TIN> v)
     return cx<T>{(T)re, (T)im};
 }
 
+template <typename T, int L>
+constexpr int strided_tb()
+{
+    // largest column tile with the FFT tile in <= 48 KB of LDS
+    constexpr int bytes = (int)sizeof(cx<T>) * L;
+    return (bytes * 16 <= 49152) ? 16 : (bytes * 8 <= 49152) ? 8 : (bytes * 4 <= 49152) ? 4 : (bytes * 2 <= 49152) ? 2 : 1;
+}
+
 // ---------------------------------------------------------------------------
 // Strided batched pass: transforms along a row dimension of [A][rows][B]
 // (B contiguous), TB consecutive columns per block.
@@ -165,22 +173,16 @@ __host__ __device__ constexpr bool sstage_fits()
 // i k transform of column b - TB, both formed from one staged tile), so the
 // next item's copy is issued after the one shared stage 0 and stays in
 // flight across both transforms; 2 the single jobs.
-// LINE: the unpruned in-place transform of the FFT_package layouts, whose rows
-// have no pitch: every staged column is checked against B (nothing outside the
-// rows is read), FP32 rows are copied 4 bytes a lane (an odd number of 8-byte
-// elements leaves them 8-byte aligned), and every twiddle factor is read from
-// the table.  An item's outputs are its own columns, which no other item reads,
-// so in place is safe with the next item's copy in flight.
-template <typename TIN, typename TOUT, typename T, int L, int TB, int NT, int DIR, bool STDP = false, int JSEL = 0, bool LINE = false>
+template <typename TIN, typename TOUT, typename T, int L, int TB, int NT, int DIR, bool STDP = false, int JSEL = 0>
 __device__ __forceinline__ void sstage_body(const StridedArgs& a)
 {
     constexpr int NB = JSEL == 1 ? 2 * TB : TB;  // columns of the transform (and LDS row pitch of fbuf)
     static_assert((TB & (TB - 1)) == 0, "column tile must be a power of two");
-    constexpr int SROWS = LINE ? L : sstage_rows<L, DIR>();
-    constexpr int SLOT = LINE && sizeof(cx<TIN>) < 16 ? 4 : 16;  // bytes per lane of a copy
-    constexpr int SPR = TB * (int)sizeof(cx<TIN>) / SLOT;        // copy slots per staged row
+    constexpr int SROWS = sstage_rows<L, DIR>();
+    constexpr int SPR = TB * (int)sizeof(cx<TIN>) / 16;  // 16-byte copy slots per staged row
+    constexpr int EPS = 16 / (int)sizeof(cx<TIN>);        // input elements per slot
     constexpr int NW = NT / 64;
-    constexpr int TWM = LINE ? 0 : sizeof(T) == 8 ? 1 : 2;
+    constexpr int TWM = sizeof(T) == 8 ? 1 : 2;
     constexpr int TWN = fft_twiddle_span<L, TWM>();  // the table entries the transform reads
     __shared__ __align__(16) cx<T> fbuf[L * NB];
     __shared__ __align__(16) cx<TIN> stg[SROWS * TB];
@@ -212,17 +214,11 @@ __device__ __forceinline__ void sstage_body(const StridedArgs& a)
         const int r = (int)(it - ai * per_a);
         const int js = r / ntiles, b0 = (r - js * ntiles) * TB;
         const int jb = (int)((jsel >> (4 * js)) & 15);
-        const char* in = (const char*)((const cx<TIN>*)a.job[jb].in + ai * a.in_a_stride + b0);
-        const int64_t rowb = a.in_row_stride * (int64_t)sizeof(cx<TIN>);
-        const int colb = LINE ? (a.B - b0) * (int)sizeof(cx<TIN>) : 0;  // bytes of this tile's rows
+        const cx<TIN>* in = (const cx<TIN>*)a.job[jb].in + ai * a.in_a_stride + b0;
         for (int m = wave; m * 64 < nslot; m += NW) {
             const int s = m * 64 + lane;
             const int row = s / SPR, part = s - row * SPR;
-            if (s < nslot && (!LINE || part * SLOT < colb)) {
-                const char* g = in + row * rowb + part * SLOT;
-                if constexpr (SLOT == 4) dma4(g, stg_base + (uint32_t)m * 256u);
-                else dma16(g, stg_base + (uint32_t)m * 1024u);
-            }
+            if (s < nslot) dma16(in + (int64_t)row * a.in_row_stride + part * EPS, stg_base + (uint32_t)m * 1024u);
         }
     };
 
@@ -325,14 +321,76 @@ __global__ __launch_bounds__(NT) void k_sstage(StridedArgs a)
     sstage_body<TIN, TOUT, T, L, TB, NT, DIR, STDP, JSEL>(a);
 }
 
-// In-place transforms of the FFT_package drop-in along y or x.  Bounded by HBM
-// (one read and one write of the field).  The direct-load kernel it replaces
-// left the memory idle while a block transformed: 768^3 FP64 2.58 -> 2.07 ms
-// (3.5 TB/s), 384^3 FP32 353 -> 132 us a pass.
+// ---------------------------------------------------------------------------
+// In-place unpruned transforms of the FFT_package drop-in along y or x, whose
+// rows have no pitch (FP32 rows start at odd multiples of 8 bytes).  Persistent
+// blocks over column tiles; a thread holds the stage-0 inputs of its butterfly,
+// loaded while the tile before is transformed, and the last stage stores to
+// global memory itself, so a block needs LDS for the transform alone and several
+// fit a CU.  A tile's outputs are its own columns, which no other tile reads, so
+// in place is safe with the next tile's loads in flight.  Every twiddle factor is
+// read from the table.  Bounded by HBM (one read and one write of the field).
+// A whole r2c, this against tiles staged in LDS (one or two blocks a CU), which
+// had taken a pass from 2.58 to 2.07 ms (768^3 FP64) and 353 to 132 us (384^3
+// FP32): 768^3 FP64 5.54 -> 4.98 ms, 384^3 FP32 351 -> 275 us, 288x144x96 FP32
+// 58 -> 47 us, 48^3 26.0 -> 21.6 us.
+// ---------------------------------------------------------------------------
+// Columns per tile: 128-byte row pieces as far as the threads (at most 1024) and
+// the LDS go.  FP32: 16 to L = 512 (there 668 us a 512^3 transform against 811
+// with 8), FP64: 8 (192^3: 76 us against 121 with 16, whose blocks have 1024
+// threads); beyond, the strided passes' tile.
+template <typename T, int L>
+__host__ __device__ constexpr int line_tb()
+{
+    constexpr int tb = strided_tb<T, L>();
+    return sizeof(T) == 4 ? (L <= 512 ? 16 : tb) : (tb < 8 ? tb : 8);
+}
+
 template <typename T, int L, int TB, int NT, int DIR>
 __global__ __launch_bounds__(NT) void k_line(StridedArgs a)
 {
-    sstage_body<T, T, T, L, TB, NT, DIR, false, 0, true>(a);
+    constexpr int R0 = Plan<L>::r(0), LR0 = L / R0;
+    static_assert(LR0 * TB <= NT, "one stage-0 butterfly a thread");
+    __shared__ __align__(16) cx<T> fbuf[L * TB];
+    __shared__ __align__(16) cx<T> twl[L];
+    const int t = threadIdx.x, b = t % TB, j = t / TB;
+    const int ntiles = (a.B + TB - 1) / TB;
+    const int64_t nitems = (int64_t)a.A * ntiles;
+    const int G = gridDim.x;  // a multiple of 8
+    cx<T>* data = (cx<T>*)a.job[0].in;
+    cx<T> in[R0];
+    // first element of an item's tile; its columns
+    auto tile = [&](int64_t it, int& ncol) -> cx<T>* {
+        const int64_t ai = it / ntiles;
+        const int b0 = (int)(it - ai * ntiles) * TB;
+        ncol = min(TB, a.B - b0);
+        return data + ai * a.in_a_stride + b0;
+    };
+    auto fetch = [&](int64_t it) {
+        int ncol;
+        const cx<T>* src = tile(it, ncol) + b;
+        if (j < LR0 && b < ncol) {
+#pragma unroll
+            for (int r = 0; r < R0; r++) in[r] = src[(int64_t)(j + r * LR0) * a.in_row_stride];
+        }
+    };
+#pragma unroll
+    for (int r = 0; r < R0; r++) in[r] = cx<T>{(T)0, (T)0};
+    int64_t it = (int64_t)(blockIdx.x % 8) * (G / 8) + blockIdx.x / 8;
+    if (it < nitems) fetch(it);
+    for (int i = t; i < L; i += NT) twl[i] = ((const cx<T>*)a.tw)[i];
+    for (; it < nitems; it += G) {
+        int ncol;
+        cx<T>* out = tile(it, ncol);
+        auto load = [&](int, int, auto rc) -> cx<T> { return in[decltype(rc)::value]; };
+        auto store = [&](int bb, int p, cx<T> v) {
+            if (bb < ncol) out[(int64_t)p * a.out_row_stride + bb] = v;
+        };
+        auto next = [&]() {
+            if (it + G < nitems) fetch(it + G);
+        };
+        FftS<T, L, TB, NT, TB, DIR, false, 0>::template run<false>(fbuf, twl, load, store, next, t);
+    }
 }
 
 template <typename TIN, typename TOUT, typename T, int L, int TB, int NT, int DIR, bool STDP = false, int JSEL = 0>
@@ -2758,14 +2816,6 @@ __global__ void k_normalize(NormArgs a)
 // ---------------------------------------------------------------------------
 // Launch tables
 // ---------------------------------------------------------------------------
-template <typename T, int L>
-constexpr int strided_tb()
-{
-    // largest column tile with the FFT tile in <= 48 KB of LDS
-    constexpr int bytes = (int)sizeof(cx<T>) * L;
-    return (bytes * 16 <= 49152) ? 16 : (bytes * 8 <= 49152) ? 8 : (bytes * 4 <= 49152) ? 4 : (bytes * 2 <= 49152) ? 2 : 1;
-}
-
 template <int L>
 constexpr int zpass_nt()
 {
@@ -3379,9 +3429,9 @@ hipError_t launch_zplain(int L, int prec, int dir, const ZPlainArgs& a, hipStrea
 template <typename T, int L, int DIR>
 static hipError_t launch_line_L(const StridedArgs& a, hipStream_t st)
 {
-    constexpr int TB = strided_tb<T, L>(), NT = sstage_nt<L, TB>();
-    static_assert(sizeof(cx<T>) * (2 * (size_t)L * TB + L) <= 160 * 1024 - 512, "tile, staging and table fit the LDS");
-    if (a.njobs != 1 || a.nin != L || a.nout != L || a.job[0].out2 || a.job[0].deriv) return hipErrorInvalidValue;
+    constexpr int TB = line_tb<T, L>(), NT = sstage_nt<L, TB>();
+    static_assert(sizeof(cx<T>) * ((size_t)L * TB + L) <= 160 * 1024 - 512, "tile and table fit the LDS");
+    if (a.njobs != 1 || a.nin != L || a.nout != L || a.job[0].out2 || a.job[0].deriv || a.job[0].in != a.job[0].out) return hipErrorInvalidValue;
     const int g = resident_grid(k_line<T, L, TB, NT, DIR>, NT, (int64_t)a.A * ((a.B + TB - 1) / TB));
     if (g < 1) return hipErrorUnknown;
     hipLaunchKernelGGL((k_line<T, L, TB, NT, DIR>), dim3(g), dim3(NT), 0, st, a);
