@@ -1300,11 +1300,14 @@ __device__ __forceinline__ void z_pair_dz(cx<T> A, int k, cx<T>& lo, cx<T>& hi)
     hi = cx<T>{b * A.x, b * -A.y};
 }
 
-// Pencils per block: whole waves of butterflies at the short lengths.
-template <int L, bool LES>
+// Pencils per block: two at the short DNS lengths, so that butterflies fill whole
+// waves (96^3 points, FP32: a run 84 us a step against 87 with one, 16 of them 654
+// against 670; four: 89 and 720), but one in FP64 at 96 and 144, where two hold
+// 126 VGPRs (16 x 64^3: 1.23 ms a step against 1.47, 64^3 alone 116 us against 125).
+template <typename T, int L, bool LES>
 __host__ __device__ constexpr int zreg_pp()
 {
-    return LES ? 1 : L <= 72 ? 4 : L <= 144 ? 2 : 1;
+    return LES ? 1 : L <= (sizeof(T) == 4 ? 144 : 72) ? 2 : 1;
 }
 
 // Threads: one butterfly each in every stage after the first (whose radix is
@@ -1333,7 +1336,7 @@ __host__ __device__ constexpr bool zreg_dzpair()
 
 template <typename T, int L, bool LES>
 struct ZReg {
-    static constexpr int PP = zreg_pp<L, LES>();
+    static constexpr int PP = zreg_pp<T, L, LES>();
     static constexpr int NI = 6 * PP, NF = (LES ? 5 : 2) * PP;
     static constexpr int NB = LES ? NI : NI + NF;
     static constexpr int NT = zreg_nt<L, NB>(LES ? PP * L : 0);
@@ -3312,10 +3315,15 @@ static int zpass_grid_L(const ZArgs& a, int64_t npen)
     constexpr int NKC = zstage_nkc<L>();
     int nb = 0;
     int64_t items = npen;
+    int min_groups = 1;
     switch (zpass_pick<T, L, 0>(a)) {
     case ZV_REG:
         nb = zreg_blocks(L, sizeof(T) == 8 ? PREC_FP64 : PREC_FP32, a.les);
-        items = npen / (a.les ? zreg_pp<L, true>() : zreg_pp<L, false>());
+        items = npen / (a.les ? zreg_pp<T, L, true>() : zreg_pp<T, L, false>());
+        // a DNS block runs one step more than it has groups (its last products),
+        // so at least two groups each, as long as every CU keeps two blocks
+        // (16 x 32^3: 125 -> 114 us a step; one run the same)
+        if (!a.les) min_groups = 2;
         break;
     case ZV_FUSE_NKC:
         if constexpr (zfuse_fits<T, L>()) nb = blocks_per_cu(k_zfuse<T, L, zfuse_nt<T, L>(), NKC>, zfuse_nt<T, L>());
@@ -3334,8 +3342,11 @@ static int zpass_grid_L(const ZArgs& a, int64_t npen)
     int dev = 0, ncu = 0;
     if (hipGetDevice(&dev) != hipSuccess) return -1;
     if (hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return -1;
-    const int64_t g = (int64_t)ncu * nb;
-    return (int)(items < g ? items : g);
+    int64_t g = (int64_t)ncu * nb;
+    if (items < g) g = items;
+    const int64_t fewer = (items + min_groups - 1) / min_groups;
+    if (fewer < g && fewer >= 2 * ncu) g = fewer;
+    return (int)g;
 }
 
 int zpass_grid(int L, int prec, const ZArgs& a, int64_t npen)
