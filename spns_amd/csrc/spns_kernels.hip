@@ -740,7 +740,9 @@ __device__ __forceinline__ void grad_invariants(const T g[9], T out[5])
 }
 
 // ---------------------------------------------------------------------------
-// z pass with the next pencil's inputs in flight (the default form).
+// z pass with the next pencil's inputs in flight: the velocity-only and
+// invariants passes, and the step where the retained k3 count is not that of the
+// 3/2 padding (else k_zreg or k_zfuse).
 // Same arithmetic as k_zpass, restructured around HBM latency:
 //   * the nine half-spectrum source fields of a pencil are staged into LDS
 //     as [field][k] (pitch SP = pitch + pad) by asynchronous global->LDS
@@ -1000,7 +1002,8 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(MINW))) void
 
 // ---------------------------------------------------------------------------
 // DNS z pass with the forward transforms of pencil n-1 folded into the
-// inverse transforms of pencil n (the default DNS form).
+// inverse transforms of pencil n (DNS from 768 points, FP32 at 288 and 384 too;
+// k_zreg elsewhere).
 // One Stockham transform of 8 columns per pencil step:
 //   columns 0-5: the six paired c2r inputs of pencil n (from the staging
 //                area, as in k_zstage);
@@ -3198,7 +3201,7 @@ constexpr int zfuse_nt()
 template <typename T, int L>
 constexpr bool zfuse_fits()
 {
-    return zstage_nkc<L>() > 0 && zfuse_lds_bytes<T, L, zfuse_nt<T, L>(), zstage_nkc<L>()>() <= 160 * 1024 - 512;
+    return !zreg_dns<T, L>() && zstage_nkc<L>() > 0 && zfuse_lds_bytes<T, L, zfuse_nt<T, L>(), zstage_nkc<L>()>() <= 160 * 1024 - 512;
 }
 
 template <typename T, int L, int MODE>
@@ -3584,9 +3587,8 @@ static int yepi_grid_L(int nbins, int nout, int A, int B, int max_grid, bool inv
     if (les ? YComb<T, L, true>::use : YComb<T, L, false>::use)
         return ycomb_grid(L, sizeof(T) == 8 ? PREC_FP64 : PREC_FP32, les, nbins, nout, A, B, max_grid);
     if (les) return 0;
-
     constexpr int TB = strided_tb<T, L>();
-    if constexpr (TB <= 0 || (TB * sizeof(cx<T>)) % 16 != 0) {
+    if constexpr (YComb<T, L, false>::use || TB <= 0 || (TB * sizeof(cx<T>)) % 16 != 0) {
         return 0;
     } else {
         if (nout > 2 * (L / 3) + 1) return 0;
@@ -3647,44 +3649,47 @@ static hipError_t launch_yepi_L(const StridedArgs& a, int A, const EpiArgs& e, i
             return launch_ycomb(L, sizeof(T) == 8 ? PREC_FP64 : PREC_FP32, b, e, grid, st, bl, ia ? &ib : nullptr, x1v);
         }
         if (e.les) return hipErrorNotSupported;
-        if (bl) {
-            constexpr int NT = yepi_nt<L, TB>();
-            const size_t shm = sizeof(double) * (NT / 64) * (size_t)e.nbins;
-            if constexpr (batch_length(L)) {
-                if (ia) {
-                    // with the next step's inverse y pass: ia is a slot's struct (all
-                    // slots share the shape class), the slots' structs are in args3
-                    bool ok = bl->args3 && ia->setflag && ia->padded_ok && ia->njobs == 3 && ia->nout == L && ia->nin == a.nout &&
-                              ia->B == a.B;
-                    for (int j = 0; ok && j < 3; j++) ok = ia->job[j].in && ia->job[j].out && ia->job[j].out2;
-                    if (!ok) return hipErrorInvalidValue;
-                    hipLaunchKernelGGL((k_yepi_inv_b<T, L, TB, NT>), dim3(grid, bl->nslots), dim3(NT), shm, st,
-                                       (const StridedArgs*)bl->args, (const EpiArgs*)bl->args2, (const StridedArgs*)bl->args3, bl->left);
+        if constexpr (!YComb<T, L, false>::use) {
+            if (bl) {
+                constexpr int NT = yepi_nt<L, TB>();
+                const size_t shm = sizeof(double) * (NT / 64) * (size_t)e.nbins;
+                if constexpr (batch_length(L)) {
+                    if (ia) {
+                        // with the next step's inverse y pass: ia is a slot's struct (all
+                        // slots share the shape class), the slots' structs are in args3
+                        bool ok = bl->args3 && ia->setflag && ia->padded_ok && ia->njobs == 3 && ia->nout == L && ia->nin == a.nout &&
+                                  ia->B == a.B;
+                        for (int j = 0; ok && j < 3; j++) ok = ia->job[j].in && ia->job[j].out && ia->job[j].out2;
+                        if (!ok) return hipErrorInvalidValue;
+                        hipLaunchKernelGGL((k_yepi_inv_b<T, L, TB, NT>), dim3(grid, bl->nslots), dim3(NT), shm, st,
+                                           (const StridedArgs*)bl->args, (const EpiArgs*)bl->args2, (const StridedArgs*)bl->args3, bl->left);
+                        return hipGetLastError();
+                    }
+                    hipLaunchKernelGGL((k_yepi_b<T, L, TB, NT>), dim3(grid, bl->nslots), dim3(NT), shm, st, (const StridedArgs*)bl->args,
+                                       (const EpiArgs*)bl->args2, bl->left);
                     return hipGetLastError();
                 }
-                hipLaunchKernelGGL((k_yepi_b<T, L, TB, NT>), dim3(grid, bl->nslots), dim3(NT), shm, st, (const StridedArgs*)bl->args,
-                                   (const EpiArgs*)bl->args2, bl->left);
+                return hipErrorNotSupported;
+            }
+            if (ia) {
+                // the inverse pass's items must be the forward pass's: same
+                // outer extent and column tiles, all rows of the transform out
+                bool ok = x1v && ia->padded_ok && ia->njobs == 3 && ia->nout == L && ia->nin == a.nout && ia->B == a.B;
+                for (int j = 0; ok && j < 3; j++) ok = ia->job[j].in && ia->job[j].out && ia->job[j].out2;
+                if (!ok) return hipErrorInvalidValue;
+                StridedArgs ib = *ia;
+                ib.A = A;
+                constexpr int NT = yepi_nt<L, TB>();
+                const size_t shm = sizeof(double) * (NT / 64) * (size_t)e.nbins;
+                hipLaunchKernelGGL((k_yepi_inv<T, L, TB, NT>), dim3(grid), dim3(NT), shm, st, b, e, ib, x1v);
                 return hipGetLastError();
             }
-            return hipErrorNotSupported;
-        }
-        if (ia) {
-            // the inverse pass's items must be the forward pass's: same
-            // outer extent and column tiles, all rows of the transform out
-            bool ok = x1v && ia->padded_ok && ia->njobs == 3 && ia->nout == L && ia->nin == a.nout && ia->B == a.B;
-            for (int j = 0; ok && j < 3; j++) ok = ia->job[j].in && ia->job[j].out && ia->job[j].out2;
-            if (!ok) return hipErrorInvalidValue;
-            StridedArgs ib = *ia;
-            ib.A = A;
             constexpr int NT = yepi_nt<L, TB>();
             const size_t shm = sizeof(double) * (NT / 64) * (size_t)e.nbins;
-            hipLaunchKernelGGL((k_yepi_inv<T, L, TB, NT>), dim3(grid), dim3(NT), shm, st, b, e, ib, x1v);
+            hipLaunchKernelGGL((k_yepi<T, L, TB, NT>), dim3(grid), dim3(NT), shm, st, b, e);
             return hipGetLastError();
         }
-        constexpr int NT = yepi_nt<L, TB>();
-        const size_t shm = sizeof(double) * (NT / 64) * (size_t)e.nbins;
-        hipLaunchKernelGGL((k_yepi<T, L, TB, NT>), dim3(grid), dim3(NT), shm, st, b, e);
-        return hipGetLastError();
+        return hipErrorNotSupported;
     }
 }
 
