@@ -1132,8 +1132,13 @@ struct spns_batch {
         slot[s] = nullptr;
         bool any = false;
         for (spns_ctx* o : slot) any = any || o;
-        if (!any) rep = nullptr;
-        else if (rep == nullptr || std::find(slot.begin(), slot.end(), rep) == slot.end())
+        if (!any) {
+            // the next context may be of another class, and the chunk's graph holds
+            // this class's kernels and grids (it is idle: the stream was waited for)
+            rep = nullptr;
+            if (graph) HIPCHK(hipGraphExecDestroy(graph));
+            graph = nullptr;
+        } else if (rep == nullptr || std::find(slot.begin(), slot.end(), rep) == slot.end())
             for (spns_ctx* o : slot) if (o) { rep = o; break; }
     }
 
@@ -1194,7 +1199,8 @@ struct spns_batch {
         HIPCHK(hipSetDevice(device));
         if (!graph) {
             // the chunk's launches read only the device arrays and counters,
-            // so one capture serves every later set of slots
+            // so one capture serves every later set of slots of the class
+            // (detach drops it with the last slot)
             hipGraph_t g;
             HIPCHK(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
             try {

@@ -1,0 +1,71 @@
+"""A batch whose last context has left takes a context of another shape class:
+its next chunk runs that class's kernels.  On the CPU the launches are compared
+with those of a new batch (tests/host_hip.py); on the GPU the results with the
+same run alone, bit for bit."""
+import os
+
+import pytest
+
+import host_hip
+
+# (N, precision, LES): each batch holds the first class, then the second
+PAIRS = [((96, 1, False), (32, 1, False)), ((32, 1, False), (32, 1, True)), ((32, 0, True), (64, 1, False))]
+
+needs_lib = pytest.mark.skipif(not os.path.exists(host_hip.LIB), reason="libspns.so not built")
+
+
+@needs_lib
+@pytest.mark.parametrize("first,second", PAIRS + [(b, a) for a, b in PAIRS])
+def test_launches_of_the_new_class(tmp_path, first, second):
+    host_hip.run(tmp_path, """
+def slot(N, prec, les):
+    s = spns_amd.Solver(Nx=N, nu=1e-3, precision=prec, C_Smag=0.17 if les else 0.0)
+    s.init_random(seed=1)
+    s.finish_init(False)
+    return s
+
+def chunk(b, s):
+    b.attach(1, s)
+    log()
+    b.step([0, 2])
+    b.synchronize()
+    return [l for l in log() if l.startswith("kernel ")]
+
+first, second = %r, %r
+runs = [slot(*first), slot(*second), slot(*second)]
+b, new = spns_amd.Batch(2, 2), spns_amd.Batch(2, 2)
+chunk(b, runs[0])
+b.detach(1)
+got, want = chunk(b, runs[1]), chunk(new, runs[2])
+assert got == want, (got, want)
+""" % (first, second))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("first,second", PAIRS)
+def test_results_of_the_new_class(first, second):
+    import numpy as np
+    import spns_amd
+
+    def slot(N, prec, les, seed):
+        s = spns_amd.Solver(Nx=N, nu=1e-3, C_At=0.5, precision=prec, C_Smag=0.17 if les else 0.0)
+        s.init_random(seed=seed, k0=4.0)
+        s.finish_init(False)
+        return s
+
+    b = spns_amd.Batch(2, 4)
+    seed = 0
+    for case in (first, second, first):
+        seed += 1
+        s, alone = slot(*case, seed), slot(*case, seed)
+        b.attach(1, s)
+        for n in (4, 3):
+            b.step([0, n])
+            alone.step(n)
+        b.synchronize()
+        assert np.array_equal(s.get_state(), alone.get_state())
+        assert np.array_equal(s.spectrum(), alone.spectrum())
+        b.detach(1)
+        s.close()
+        alone.close()
+    b.close()
