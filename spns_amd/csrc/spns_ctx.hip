@@ -1122,7 +1122,8 @@ struct spns_batch {
         HIPCHK(hipEventRecord(ev_sc, st));
         HIPCHK(hipEventRecord(ev, st));
         slot[s] = c;
-        rep = r ? r : c;
+        // r may be the context that c replaces here, and then go away
+        rep = r && std::find(slot.begin(), slot.end(), r) != slot.end() ? r : c;
     }
 
     void detach(int s)

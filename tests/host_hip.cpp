@@ -12,6 +12,8 @@
 #include <string>
 #include <vector>
 
+#include <malloc.h>
+
 #include <hip/hip_runtime_api.h>
 
 namespace {
@@ -41,8 +43,14 @@ void* operator new(size_t n)
     if (!p) throw std::bad_alloc();
     return p;
 }
-void operator delete(void* p) noexcept { std::free(p); }
-void operator delete(void* p, size_t) noexcept { std::free(p); }
+// freed objects are overwritten, so that a later use shows
+void operator delete(void* p) noexcept
+{
+    if (p) std::memset(p, 0xdd, malloc_usable_size(p));
+    asm volatile("" ::"r"(p) : "memory");  // or the fill is dropped as dead
+    std::free(p);
+}
+void operator delete(void* p, size_t) noexcept { operator delete(p); }
 
 extern "C" {
 // for the tests

@@ -41,6 +41,19 @@ assert got == want, (got, want)
 """ % (first, second))
 
 
+@needs_lib
+def test_replaced_context_gives_the_class_no_more(tmp_path):
+    host_hip.run(tmp_path, """
+a, b, c = [spns_amd.Solver(Nx=32, nu=1e-3, precision=1) for _ in range(3)]
+batch = spns_amd.Batch(2, 2)
+batch.attach(0, a)
+batch.attach(0, b)  # takes a's place
+a.close()
+batch.attach(1, c)
+batch.step([1, 1])
+""")
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("first,second", PAIRS)
 def test_results_of_the_new_class(first, second):
