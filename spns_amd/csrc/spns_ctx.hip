@@ -1268,9 +1268,31 @@ thread_local std::string g_create_error;
 
 }  // namespace
 
+// A call works on the context's device whichever is the calling thread's current
+// one (kernel launches and new events take that one), and leaves that as it was.
+namespace {
+struct OnDevice {
+    int was = -1;
+    explicit OnDevice(int device)
+    {
+        int cur = 0;
+        HIPCHK(hipGetDevice(&cur));
+        if (cur == device) return;
+        HIPCHK(hipSetDevice(device));
+        was = cur;
+    }
+    OnDevice(const OnDevice&) = delete;
+    ~OnDevice()
+    {
+        if (was >= 0) (void)hipSetDevice(was);
+    }
+};
+}  // namespace
+
 #define API_BEGIN(c) \
     if (!(c)) return SPNS_EINVAL; \
-    try {
+    try { \
+        const OnDevice on_device((c)->cfg.device);
 #define API_END(c)                                   \
     }                                                \
     catch (const Error& e) { return finish(c, e, e.code); } \
@@ -1306,7 +1328,6 @@ int spns_reconfigure(spns_ctx* ctx, const spns_config* cfg)
 {
     API_BEGIN(ctx)
     if (!cfg) throw Error(SPNS_EINVAL, "null config");
-    HIPCHK(hipSetDevice(ctx->cfg.device));
     ctx->x1_stale();  // the state changes
     ctx->reconfigure(*cfg);
     API_END(ctx)
@@ -1348,7 +1369,6 @@ int spns_set_state(spns_ctx* ctx, const double* state)
     API_BEGIN(ctx)
     ctx->x1_stale();  // the state changes
     if (!state) throw Error(SPNS_EINVAL, "null state");
-    HIPCHK(hipSetDevice(ctx->cfg.device));
     ctx->upload_state(state);
     API_END(ctx)
 }
@@ -1652,7 +1672,6 @@ int spns_get_scalars(spns_ctx* ctx, spns_scalars* out)
 static void physical_out(spns_ctx* ctx, double* uvw, bool step_start)
 {
     if (!uvw) throw Error(SPNS_EINVAL, "null output");
-    HIPCHK(hipSetDevice(ctx->cfg.device));
     const size_t P = (size_t)ctx->Mx * ctx->My * ctx->Mz, pb = sizeof(double) * P;
     char* room[2] = {(char*)ctx->X2f(3), (char*)ctx->X1};
     size_t left[2] = {(size_t)6 * ctx->x2_slot * ctx->tsz, (size_t)ctx->n_x1 * ctx->x1_slot * ctx->tsz};
@@ -1820,7 +1839,6 @@ int spns_invariant_spectra_noalloc(spns_ctx* ctx, int32_t nbins, double* spectra
                                      std::to_string(kNoAllocScratchDoubles) + " (use spns_invariant_spectra)");
     if (!ctx->scratch_dev)
         throw Error(SPNS_EHIP, std::string("hipGetSymbolAddress(scratch): ") + hipGetErrorString(ctx->scratch_err));
-    HIPCHK(hipSetDevice(ctx->cfg.device));
     ctx->invariant_spectra_dev(ctx->scratch_dev);
     HIPCHK(hipMemcpy2DAsync(spectra, sizeof(double) * nbins, ctx->scratch_dev, sizeof(double) * ctx->nbins,
                             sizeof(double) * ctx->nbins, 5, hipMemcpyDeviceToHost, ctx->st));

@@ -21,6 +21,7 @@ std::mutex mu;
 std::string text;                       // one line per operation that ran
 std::map<const void*, std::string> names;
 thread_local int current = 0;
+thread_local hipError_t last = hipSuccess;
 thread_local long fail_alloc = -1;      // allocations until one throws; < 0: none does
 struct Stream { int dev; std::vector<std::string>* capture = nullptr; };
 struct Event { int dev; };
@@ -73,7 +74,7 @@ hipError_t __hipPopCallConfiguration(dim3* g, dim3* b, size_t* shm, hipStream_t*
 }
 hipError_t hipLaunchKernel(const void* f, dim3 g, dim3 b, void**, size_t, hipStream_t s)
 {
-    if (of(s)->dev != current) return hipErrorInvalidHandle;
+    if (of(s)->dev != current) return last = hipErrorInvalidHandle;
     note(s, "kernel " + names[f] + " " + std::to_string(g.x) + "x" + std::to_string(g.y) + " " + std::to_string(b.x));
     return hipSuccess;
 }
@@ -96,7 +97,12 @@ hipError_t hipOccupancyMaxActiveBlocksPerMultiprocessor(int* n, const void*, int
 }
 hipError_t hipFuncGetAttributes(hipFuncAttributes* a, const void*) { std::memset(a, 0, sizeof *a); return hipSuccess; }
 hipError_t hipGetSymbolAddress(void** p, const void*) { *p = nullptr; return hipErrorInvalidSymbol; }
-hipError_t hipGetLastError() { return hipSuccess; }
+hipError_t hipGetLastError()
+{
+    const hipError_t e = last;
+    last = hipSuccess;
+    return e;
+}
 const char* hipGetErrorString(hipError_t e) { return e == hipSuccess ? "no error" : "error"; }
 
 hipError_t hipMalloc(void** p, size_t n) { *p = std::calloc(n ? n : 1, 1); return *p ? hipSuccess : hipErrorOutOfMemory; }
