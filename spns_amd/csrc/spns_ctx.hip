@@ -105,6 +105,9 @@ void check_strided(StridedArgs& a, int A, const int64_t* in_cap, const int64_t* 
 // the page faults and the host's own copy are serial; this moves 32 (52 and
 // 170 MB; six or eight threads the same).  Small ones are one hipMemcpy: below
 // kSmall the threads cost more than they save.
+// A Piece is the device side: move queues the copy of its bytes [off, off + n) from
+// or to pinned memory on st, move_by that from or to any host memory, by way of
+// device memory of its owner (room, kSmall bytes) where it has to.
 // The pinned memory (16 MiB) belongs to the owner and goes with it.
 // ===========================================================================
 namespace {
@@ -115,12 +118,16 @@ struct HostCopy {
     hipEvent_t ev[kThreads][2] = {};
 
     // Complete on return.  Work queued on st before the call is finished first.
-    void copy(void* host, void* devp, size_t bytes, bool to_host, int device, hipStream_t st)
+    template <class Piece>
+    void copy(void* host, size_t bytes, int device, hipStream_t st, const Piece& piece, char* room = nullptr)
     {
-        const hipMemcpyKind kind = to_host ? hipMemcpyDeviceToHost : hipMemcpyHostToDevice;
+        constexpr bool to_host = Piece::to_host;
         if (bytes < kSmall || !ready()) {
-            if (to_host) HIPCHK(hipMemcpyAsync(host, devp, bytes, kind, st));
-            else HIPCHK(hipMemcpyAsync(devp, host, bytes, kind, st));
+            for (size_t off = 0; off < bytes; off += kSmall) {
+                const size_t n = std::min(kSmall, bytes - off);
+                char* h = (char*)host + off;
+                HIPCHK(piece.move_by(h, off, n, room, st));
+            }
             HIPCHK(hipStreamSynchronize(st));
             return;
         }
@@ -140,9 +147,8 @@ struct HostCopy {
             for (size_t c = w; c < nchunk && e == hipSuccess; c += kThreads, b ^= 1) {
                 drain(b);
                 if (e != hipSuccess) break;
-                char* d = (char*)devp + c * kChunk;
                 if (!to_host) std::memcpy(buf(w, b), (const char*)host + c * kChunk, size(c));
-                e = to_host ? hipMemcpyAsync(buf(w, b), d, size(c), kind, st) : hipMemcpyAsync(d, buf(w, b), size(c), kind, st);
+                e = piece.move(buf(w, b), c * kChunk, size(c), st);
                 if (e == hipSuccess) e = hipEventRecord(ev[w][b], st);
                 if (e == hipSuccess) pend[b] = c;
             }
@@ -197,6 +203,42 @@ struct HostCopy {
             }
         if (pin) hipHostFree(pin);
         pin = nullptr;
+    }
+};
+}  // namespace
+
+namespace {
+// contiguous device memory
+template <bool OUT>
+struct PlainPiece {
+    static constexpr bool to_host = OUT;
+    char* d;
+    hipError_t move(char* h, size_t off, size_t n, hipStream_t st) const
+    {
+        return OUT ? hipMemcpyAsync(h, d + off, n, hipMemcpyDeviceToHost, st) : hipMemcpyAsync(d + off, h, n, hipMemcpyHostToDevice, st);
+    }
+    hipError_t move_by(char* h, size_t off, size_t n, char*, hipStream_t st) const { return move(h, off, n, st); }
+};
+
+// the compact box of pitched fields, outwards.  The kernel writes pinned memory
+// itself: 192^3 (173 MB) 3.6 ms against 4.4 packed and copied, and 5.0 with a
+// pack and a copy per chunk.
+struct PackPiece {
+    static constexpr bool to_host = true;
+    PackArgs a;
+    bool fp32;
+    hipError_t move(char* h, size_t off, size_t n, hipStream_t st) const
+    {
+        PackArgs p = a;
+        p.compact = (cx<double>*)h;
+        p.first = (int64_t)(off / sizeof(cx<double>));
+        p.n = (uint32_t)(n / sizeof(cx<double>));
+        return launch_pack(p, fp32, st);
+    }
+    hipError_t move_by(char* h, size_t off, size_t n, char* room, hipStream_t st) const
+    {
+        const hipError_t e = move(room, off, n, st);
+        return e != hipSuccess ? e : hipMemcpyAsync(h, room, n, hipMemcpyDeviceToHost, st);
     }
 };
 }  // namespace
@@ -340,6 +382,8 @@ struct spns_ctx {
     hipGraphExec_t graph[2] = {};
     bool x1_cur = false;
     HostCopy hcopy;
+    char* room = nullptr;  // of small packed copies: a read of the state uses none of the passes' arrays
+    std::mutex mu;         // held by every call that uses the passes' arrays, hcopy or room
     std::string err;
     double last_ms = 0.0;
 
@@ -438,6 +482,7 @@ struct spns_ctx {
         alloc((void**)&x1v, sizeof(int));
         alloc((void**)&ek, sizeof(double) * nbins);
         alloc((void**)&ft, sizeof(double) * (nbins + 1));
+        alloc((void**)&room, std::min(HostCopy::kSmall, pack_bytes((int64_t)nk2 * nk1)));
         HIPCHK(hipMemsetAsync(z_partial, 0, sizeof(double) * 4 * grid_z, st));
         HIPCHK(hipMemsetAsync(X1, 0, (size_t)n_x1 * x1_slot * tsz, st));
         HIPCHK(hipMemsetAsync(X2, 0, (size_t)9 * x2_slot * tsz, st));
@@ -533,7 +578,7 @@ struct spns_ctx {
         for (int c = 0; c < 3; c++) { hipFree(uk[c]); hipFree(R[c]); hipFree(ukprev[c]); }
         hipFree(X1); hipFree(X2); hipFree(twx); hipFree(twy); hipFree(twz);
         hipFree(scal); hipFree(hist_partial); hipFree(om_partial); hipFree(ed_partial); hipFree(z_partial); hipFree(ticket);
-        hipFree(x1v);
+        hipFree(x1v); hipFree(room);
         hipFree(ek); hipFree(forced); hipFree(ft); hipFree(invspec);
         if (ev0) hipEventDestroy(ev0);
         if (ev1) hipEventDestroy(ev1);
@@ -898,18 +943,15 @@ struct spns_ctx {
         HIPCHK(hipStreamSynchronize(st));
     }
 
-    // Compact rows [row0, row0 + nrow) of three pitched fields, packed in X2's
-    // space (free between passes; it holds all of them: retained modes fit the grid)
-    PackArgs pack_args(void* const* f, int64_t row0, int64_t nrow)
+    // Compact rows [row0, row0 + nrow) of three pitched fields
+    PackArgs pack_args(void* const* f, int64_t row0, int64_t nrow) const
     {
         PackArgs p{};
         for (int c = 0; c < 3; c++) p.padded[c] = f[c];
-        p.compact = (cx<double>*)X2;
         p.row0 = (uint32_t)row0; p.nrow = (uint32_t)nrow; p.nk3 = (uint32_t)nk3; p.nk3p = (uint32_t)nk3p;
         p.nk1 = nk1; p.nk2 = nk2;
         p.notcubic = cfg.isNotCubic; p.Lx = cfg.Lx; p.Ly = cfg.Ly; p.Lz = cfg.Lz;
-        if (row0 < 0 || nrow < 0 || row0 + nrow > (int64_t)nk2 * nk1 || pack_bytes(nrow) > (size_t)9 * x2_slot * tsz)
-            throw Error(SPNS_EINVAL, "packed state exceeds its buffer");
+        if (row0 < 0 || nrow < 0 || row0 + nrow > (int64_t)nk2 * nk1) throw Error(SPNS_EINVAL, "rows outside the state");
         return p;
     }
     size_t pack_bytes(int64_t nrow) const { return sizeof(cx<double>) * 3 * (size_t)nrow * nk3; }
@@ -918,9 +960,16 @@ struct spns_ctx {
     void upload_state(const void* h)
     {
         const int64_t rows = (int64_t)nk2 * nk1;
-        const PackArgs p = pack_args((void* const*)uk, 0, rows);
-        hcopy.copy(const_cast<void*>(h), p.compact, pack_bytes(rows), false, cfg.device, st);
-        HIPCHK(launch_unpack(p, st));
+        PackArgs p = pack_args((void* const*)uk, 0, rows);
+        if (pack_bytes(rows) > (size_t)9 * x2_slot * tsz) throw Error(SPNS_EINVAL, "packed state exceeds its buffer");
+        // by way of X2, free between passes (a state that comes in ends what a step left)
+        hcopy.copy(const_cast<void*>(h), pack_bytes(rows), cfg.device, st, PlainPiece<false>{(char*)X2});
+        p.n = (uint32_t)nmodes;
+        for (int c = 0; c < 3; c++) {
+            p.first = c * nmodes;
+            p.compact = (cx<double>*)X2 + p.first;
+            HIPCHK(launch_unpack(p, st));
+        }
         reset_history();
     }
 
@@ -940,9 +989,8 @@ struct spns_ctx {
     void download(void* const* f, bool fp32, int64_t row0, int64_t nrow, void* out)
     {
         if (nrow == 0) return;
-        const PackArgs p = pack_args(f, row0, nrow);
-        HIPCHK(launch_pack(p, fp32, st));
-        hcopy.copy(out, p.compact, pack_bytes(nrow), true, cfg.device, st);
+        const PackPiece p{pack_args(f, row0, nrow), fp32};
+        hcopy.copy(out, pack_bytes(nrow), cfg.device, st, p, room);
     }
 
     int64_t compact_index(int k1, int k2, int k3) const
@@ -1025,6 +1073,9 @@ struct spns_batch {
     EpiArgs* d_epi = nullptr;
     FinArgs* d_fin = nullptr;
     int* d_left = nullptr;
+    static constexpr size_t kRoom = 16u << 20;
+    char* room = nullptr;  // packed states on their way out
+    std::mutex mu;         // held while a fetch queues its packs and copies
     hipGraphExec_t graph = nullptr;
     std::string err;
 
@@ -1052,6 +1103,7 @@ struct spns_batch {
         al((void**)&d_z, sizeof(ZArgs) * n); al((void**)&d_epi, sizeof(EpiArgs) * n);
         al((void**)&d_fin, sizeof(FinArgs) * n);
         al((void**)&d_left, sizeof(int) * n);
+        al((void**)&room, kRoom);
         SlotSteps z{};
         HIPCHK(launch_set_left(d_left, z, nslots, st));
         HIPCHK(hipStreamSynchronize(st));
@@ -1062,7 +1114,7 @@ struct spns_batch {
         if (st) hipStreamSynchronize(st);
         if (graph) hipGraphExecDestroy(graph);
         hipFree(d_invy); hipFree(d_invx); hipFree(d_fwdx); hipFree(d_fwdy); hipFree(d_invy2); hipFree(d_z); hipFree(d_epi);
-        hipFree(d_fin); hipFree(d_left);
+        hipFree(d_fin); hipFree(d_left); hipFree(room);
         if (hs) hipHostFree(hs);
         if (hsc) hipHostFree(hsc);
         if (ev) hipEventDestroy(ev);
@@ -1245,11 +1297,14 @@ struct spns_batch {
         if (s < 0 || s >= nslots || !slot[s]) throw Error(SPNS_EINVAL, "no context in this slot");
         spns_ctx* c = slot[s];
         if (state) {
-            // packed on the batch's stream: the slot's X2 is free between chunks
+            // piece by piece through the batch's room: each pack follows the copy
+            // before it on the stream
+            const std::lock_guard<std::mutex> lk(mu);
             const int64_t rows = (int64_t)c->nk2 * c->nk1;
-            const PackArgs p = c->pack_args((void* const*)c->uk, 0, rows);
-            HIPCHK(launch_pack(p, false, st));
-            HIPCHK(hipMemcpyAsync(state, p.compact, c->pack_bytes(rows), hipMemcpyDeviceToHost, st));
+            const PackPiece p{c->pack_args((void* const*)c->uk, 0, rows), false};
+            const size_t bytes = c->pack_bytes(rows);
+            for (size_t off = 0; off < bytes; off += kRoom)
+                HIPCHK(p.move_by((char*)state + off, off, std::min(kRoom, bytes - off), room, st));
         }
         if (ek) HIPCHK(hipMemcpyAsync(ek, c->ek, sizeof(double) * c->nbins, hipMemcpyDeviceToHost, st));
         HIPCHK(hipEventRecord(ev, st));
@@ -1290,6 +1345,13 @@ struct OnDevice {
 }  // namespace
 
 #define API_BEGIN(c) \
+    if (!(c)) return SPNS_EINVAL; \
+    try { \
+        const std::lock_guard<std::mutex> one_call((c)->mu); \
+        const OnDevice on_device((c)->cfg.device);
+// for calls that use no memory of the context but its scalars and spectrum: they
+// do not wait for another thread's call
+#define API_OPEN(c) \
     if (!(c)) return SPNS_EINVAL; \
     try { \
         const OnDevice on_device((c)->cfg.device);
@@ -1587,7 +1649,7 @@ int spns_forcing_reynolds_lambda(spns_ctx* ctx, double relambda)
 
 int spns_recalculate_reynolds_lambda(spns_ctx* ctx, double* relambda)
 {
-    API_BEGIN(ctx)
+    API_OPEN(ctx)
     DevScalars s = ctx->read_scalars();
     double r = s.ek / s.nu * std::sqrt(20.0 / 3.0 / s.om);
     if (relambda) *relambda = r;
@@ -1614,7 +1676,7 @@ int spns_complex_conjugate_correction(spns_ctx* ctx)
 
 int spns_energy_cascade(spns_ctx* ctx, double* ekh, int32_t nbins, double* ek_tot)
 {
-    API_BEGIN(ctx)
+    API_OPEN(ctx)
     if (ekh && nbins > ctx->nbins) throw Error(SPNS_EINVAL, "nbins exceeds the spectrum");
     if (ekh && nbins > 0) {
         HIPCHK(hipMemcpyAsync(ekh, ctx->ek, sizeof(double) * nbins, hipMemcpyDeviceToHost, ctx->st));
@@ -1659,7 +1721,7 @@ int spns_pass_kernels(spns_ctx* ctx, int32_t* zpass_kernel, int32_t* fused_epilo
 
 int spns_get_scalars(spns_ctx* ctx, spns_scalars* out)
 {
-    API_BEGIN(ctx)
+    API_OPEN(ctx)
     if (!out) throw Error(SPNS_EINVAL, "null output");
     to_scalars(ctx, ctx->read_scalars(), out);
     API_END(ctx)
@@ -1692,7 +1754,7 @@ static void physical_out(spns_ctx* ctx, double* uvw, bool step_start)
         }
         if (step_start) ctx->velocity_step_start(d);
         else ctx->velocity_pass(d);
-        for (int c = 0; c < 3; c++) ctx->hcopy.copy(uvw + c * P, d[c], pb, true, ctx->cfg.device, ctx->st);
+        for (int c = 0; c < 3; c++) ctx->hcopy.copy(uvw + c * P, pb, ctx->cfg.device, ctx->st, PlainPiece<true>{(char*)d[c]});
     } catch (...) {
         hipStreamSynchronize(ctx->st);
         for (void* p : own) hipFree(p);
@@ -1741,14 +1803,14 @@ int spns_recalculate_velocity_antitransform(spns_ctx* ctx)
 
 int spns_synchronize(spns_ctx* ctx)
 {
-    API_BEGIN(ctx)
+    API_OPEN(ctx)
     HIPCHK(hipStreamSynchronize(ctx->st));
     API_END(ctx)
 }
 
 int spns_query(spns_ctx* ctx, int32_t* done)
 {
-    API_BEGIN(ctx)
+    API_OPEN(ctx)
     if (!done) throw Error(SPNS_EINVAL, "done is null");
     const hipError_t e = hipEventQuery(ctx->ev1);
     if (e == hipErrorNotReady) {
@@ -1897,7 +1959,7 @@ int spns_profile_passes(spns_ctx* ctx, int32_t nsteps, double* ms)
 
 int spns_last_step_ms(spns_ctx* ctx, double* ms)
 {
-    API_BEGIN(ctx)
+    API_OPEN(ctx)
     HIPCHK(hipEventSynchronize(ctx->ev1));
     float f = 0.f;
     HIPCHK(hipEventElapsedTime(&f, ctx->ev0, ctx->ev1));

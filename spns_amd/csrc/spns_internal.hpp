@@ -127,10 +127,13 @@ struct ShellArgs {
 };
 
 // Compact box (the C ABI's [c][i2][i1][i3], FP64) to or from the pitched device
-// fields, rows [row0, row0 + nrow) of the (i2, i1) rows.
+// fields, rows [row0, row0 + nrow) of the (i2, i1) rows: elements
+// [first, first + n) of [3][nrow][nk3].
 struct PackArgs {
     void* padded[3];  // cx<double>, or cx<float> (pack only: widened)
-    cx<double>* compact;  // [3][nrow][nk3]
+    cx<double>* compact;  // element `first` of the box
+    int64_t first;
+    uint32_t n;
     uint32_t row0, nrow, nk3, nk3p;
     int nk1, nk2;
     int notcubic, Lx, Ly, Lz;  // unpack: modes masked by the length factors are zeroed

@@ -2711,33 +2711,45 @@ __global__ __launch_bounds__(256) void k_stream_copy(const vf4* __restrict__ in,
 // nk3 modes leave the pitch here, on the device, so that what crosses the host
 // link is one contiguous copy: a strided copy to pageable memory moved row by
 // row (6.7 us each: 350 ms for a 128^3 state of 52 MB, and 460 ms inwards).
-// Bounded by HBM: one read and one write of the state, 0.03 ms there.
+// Bounded by HBM: one read and one write of the state, 0.03 ms there.  A launch
+// takes one piece of the box; its contiguous side is device or pinned memory.
+
+// Element i of the launch: its field, row and k3.
+static __device__ __forceinline__ void pack_element(const PackArgs& a, uint32_t i, uint32_t& c, uint32_t& r, uint32_t& k3)
+{
+    const uint32_t per = a.nrow * a.nk3;  // < 2^31 (the launcher's check)
+    const uint64_t e = (uint64_t)a.first + i;
+    c = e >= 2ull * per ? 2 : e >= per ? 1 : 0;
+    const uint32_t q = (uint32_t)(e - (uint64_t)c * per);
+    r = q / a.nk3;
+    k3 = q - r * a.nk3;
+    r += a.row0;
+}
+
 template <typename TS>
 __global__ __launch_bounds__(256) void k_pack(PackArgs a)
 {
-    const uint32_t n = a.nrow * a.nk3;
-    const cx<TS>* __restrict__ in = (const cx<TS>*)a.padded[blockIdx.y] + (int64_t)a.row0 * a.nk3p;
-    cx<double>* __restrict__ out = a.compact + (int64_t)blockIdx.y * n;
-    for (uint32_t e = blockIdx.x * 256u + threadIdx.x; e < n; e += gridDim.x * 256u) {
-        const uint32_t r = e / a.nk3;
-        const cx<TS> v = in[(int64_t)r * a.nk3p + (e - r * a.nk3)];
-        out[e] = cx<double>{(double)v.x, (double)v.y};
+    for (uint32_t i = blockIdx.x * 256u + threadIdx.x; i < a.n; i += gridDim.x * 256u) {
+        uint32_t c, r, k3;
+        pack_element(a, i, c, r, k3);
+        const cx<TS>* in = (const cx<TS>*)(c == 0 ? a.padded[0] : c == 1 ? a.padded[1] : a.padded[2]);
+        const cx<TS> v = in[(int64_t)r * a.nk3p + k3];
+        a.compact[i] = cx<double>{(double)v.x, (double)v.y};
     }
 }
 
 static __global__ __launch_bounds__(256) void k_unpack(PackArgs a)
 {
-    const uint32_t n = a.nrow * a.nk3;
-    cx<double>* __restrict__ out = (cx<double>*)a.padded[blockIdx.y] + (int64_t)a.row0 * a.nk3p;
-    const cx<double>* __restrict__ in = a.compact + (int64_t)blockIdx.y * n;
-    for (uint32_t e = blockIdx.x * 256u + threadIdx.x; e < n; e += gridDim.x * 256u) {
-        const uint32_t r = e / a.nk3, k3 = e - r * a.nk3;
-        cx<double> v = in[e];
+    for (uint32_t i = blockIdx.x * 256u + threadIdx.x; i < a.n; i += gridDim.x * 256u) {
+        uint32_t c, r, k3;
+        pack_element(a, i, c, r, k3);
+        cx<double> v = a.compact[i];
         if (a.notcubic) {  // src/HIT_LES.cpp:867-871
-            const int row = (int)(a.row0 + r), i2 = row / a.nk1;
+            const int row = (int)r, i2 = row / a.nk1;
             const int k1 = wrap_k(row - i2 * a.nk1, a.nk1), k2 = wrap_k(i2, a.nk2);
             if ((k1 % a.Lx) || (k2 % a.Ly) || ((int)k3 % a.Lz)) v = cx<double>{0.0, 0.0};
         }
+        cx<double>* out = (cx<double>*)(c == 0 ? a.padded[0] : c == 1 ? a.padded[1] : a.padded[2]);
         out[(int64_t)r * a.nk3p + k3] = v;
     }
 }
@@ -3750,21 +3762,21 @@ hipError_t launch_stream_copy(const void* in, void* out, int64_t bytes, int bloc
     return hipGetLastError();
 }
 
-// grid of the pack kernels: 0 if the rows exceed their 32-bit index
+// grid of the pack kernels: 0 if the elements exceed the box or a field their 32-bit index
 static unsigned pack_grid(const PackArgs& a)
 {
-    const int64_t n = (int64_t)a.nrow * a.nk3;
-    if (n >= ((int64_t)1 << 31)) return 0;
-    const int64_t g = (n + 255) / 256;
-    return (unsigned)(g < 8192 ? (g > 0 ? g : 1) : 8192);
+    const int64_t per = (int64_t)a.nrow * a.nk3;
+    if (per >= ((int64_t)1 << 31) || a.n < 1 || a.n >= (1u << 31) || a.first < 0 || a.first + a.n > 3 * per) return 0;
+    const uint32_t g = (a.n + 255) / 256;
+    return g < 8192 ? g : 8192;
 }
 
 hipError_t launch_pack(const PackArgs& a, bool from_fp32, hipStream_t st)
 {
     const unsigned g = pack_grid(a);
     if (!g) return hipErrorInvalidValue;
-    if (from_fp32) hipLaunchKernelGGL((k_pack<float>), dim3(g, 3), dim3(256), 0, st, a);
-    else hipLaunchKernelGGL((k_pack<double>), dim3(g, 3), dim3(256), 0, st, a);
+    if (from_fp32) hipLaunchKernelGGL((k_pack<float>), dim3(g), dim3(256), 0, st, a);
+    else hipLaunchKernelGGL((k_pack<double>), dim3(g), dim3(256), 0, st, a);
     return hipGetLastError();
 }
 
@@ -3772,7 +3784,7 @@ hipError_t launch_unpack(const PackArgs& a, hipStream_t st)
 {
     const unsigned g = pack_grid(a);
     if (!g) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(k_unpack, dim3(g, 3), dim3(256), 0, st, a);
+    hipLaunchKernelGGL(k_unpack, dim3(g), dim3(256), 0, st, a);
     return hipGetLastError();
 }
 

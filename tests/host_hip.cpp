@@ -20,6 +20,7 @@ namespace {
 std::mutex mu;
 std::string text;                       // one line per operation that ran
 std::map<const void*, std::string> names;
+std::map<char*, size_t> blocks;  // device memory
 thread_local int current = 0;
 thread_local hipError_t last = hipSuccess;
 thread_local long fail_alloc = -1;      // allocations until one throws; < 0: none does
@@ -33,6 +34,15 @@ void note(hipStream_t s, const std::string& line)
     std::lock_guard<std::mutex> lk(mu);
     if (of(s)->capture) of(s)->capture->push_back(line);
     else text += line + "\n";
+}
+// size of the device block that holds p, 0 for host memory
+size_t block_of(const void* p)
+{
+    std::lock_guard<std::mutex> lk(mu);
+    auto it = blocks.upper_bound((char*)p);
+    if (it == blocks.begin()) return 0;
+    --it;
+    return (char*)p < it->first + it->second ? it->second : 0;
 }
 void count(const char* call) { note(nullptr, std::string("call ") + call); }
 }  // namespace
@@ -105,12 +115,30 @@ hipError_t hipGetLastError()
 }
 const char* hipGetErrorString(hipError_t e) { return e == hipSuccess ? "no error" : "error"; }
 
-hipError_t hipMalloc(void** p, size_t n) { *p = std::calloc(n ? n : 1, 1); return *p ? hipSuccess : hipErrorOutOfMemory; }
-hipError_t hipFree(void* p) { std::free(p); return hipSuccess; }
-hipError_t hipHostMalloc(void** p, size_t n, unsigned) { return hipMalloc(p, n); }
-hipError_t hipHostFree(void* p) { return hipFree(p); }
+hipError_t hipHostMalloc(void** p, size_t n, unsigned) { *p = std::calloc(n ? n : 1, 1); return *p ? hipSuccess : hipErrorOutOfMemory; }
+hipError_t hipHostFree(void* p) { std::free(p); return hipSuccess; }
+hipError_t hipMalloc(void** p, size_t n)
+{
+    const hipError_t e = hipHostMalloc(p, n, 0);
+    std::lock_guard<std::mutex> lk(mu);
+    blocks[(char*)*p] = n;
+    return e;
+}
+hipError_t hipFree(void* p)
+{
+    {
+        std::lock_guard<std::mutex> lk(mu);
+        blocks.erase((char*)p);
+    }
+    return hipHostFree(p);
+}
 hipError_t hipMemcpy(void* d, const void* s, size_t n, hipMemcpyKind) { std::memcpy(d, s, n); return hipSuccess; }
-hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, hipMemcpyKind, hipStream_t) { std::memcpy(d, s, n); return hipSuccess; }
+hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, hipMemcpyKind, hipStream_t st)
+{
+    note(st, "copy " + std::to_string(n) + " to " + std::to_string(block_of(d)) + " from " + std::to_string(block_of(s)));
+    std::memcpy(d, s, n);
+    return hipSuccess;
+}
 hipError_t hipMemcpy2DAsync(void* d, size_t dp, const void* s, size_t sp, size_t w, size_t h, hipMemcpyKind, hipStream_t)
 {
     for (size_t i = 0; i < h; i++) std::memcpy((char*)d + i * dp, (const char*)s + i * sp, w);
