@@ -11,7 +11,6 @@
 #include <mutex>
 #include <stdexcept>
 #include <string>
-#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -160,8 +159,8 @@ struct HostCopy {
         for (int w = 1; w < kThreads; w++) {
             try {
                 th[w] = std::thread(work, w);
-            } catch (const std::system_error&) {
-            }  // no thread to be had: its share is done below
+            } catch (const std::exception&) {
+            }  // no thread to be had, or no memory for it: its share is done below
         }
         work(0);
         for (int w = 1; w < kThreads; w++) {

@@ -23,7 +23,12 @@ std::map<const void*, std::string> names;
 std::map<char*, size_t> blocks;  // device memory
 thread_local int current = 0;
 thread_local hipError_t last = hipSuccess;
-thread_local long fail_alloc = -1;      // allocations until one throws; < 0: none does
+thread_local long fail_alloc = -1;      // the library's allocations until one throws; < 0: none does
+thread_local bool inside = false;       // in a call below, whose own allocations do not count
+struct Inside {
+    Inside() { inside = true; }
+    ~Inside() { inside = false; }
+};
 struct Stream { int dev; std::vector<std::string>* capture = nullptr; };
 struct Event { int dev; };
 Stream null_stream{0};
@@ -44,12 +49,12 @@ size_t block_of(const void* p)
     --it;
     return (char*)p < it->first + it->second ? it->second : 0;
 }
-void count(const char* call) { note(nullptr, std::string("call ") + call); }
+void count(const char* call) { const Inside in; note(nullptr, std::string("call ") + call); }
 }  // namespace
 
 void* operator new(size_t n)
 {
-    if (fail_alloc >= 0 && fail_alloc-- == 0) throw std::bad_alloc();
+    if (!inside && fail_alloc >= 0 && fail_alloc-- == 0) throw std::bad_alloc();
     void* p = std::malloc(n ? n : 1);
     if (!p) throw std::bad_alloc();
     return p;
@@ -85,6 +90,7 @@ hipError_t __hipPopCallConfiguration(dim3* g, dim3* b, size_t* shm, hipStream_t*
 hipError_t hipLaunchKernel(const void* f, dim3 g, dim3 b, void**, size_t, hipStream_t s)
 {
     if (of(s)->dev != current) return last = hipErrorInvalidHandle;
+    const Inside in;
     note(s, "kernel " + names[f] + " " + std::to_string(g.x) + "x" + std::to_string(g.y) + " " + std::to_string(b.x));
     return hipSuccess;
 }
@@ -135,6 +141,7 @@ hipError_t hipFree(void* p)
 hipError_t hipMemcpy(void* d, const void* s, size_t n, hipMemcpyKind) { std::memcpy(d, s, n); return hipSuccess; }
 hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, hipMemcpyKind, hipStream_t st)
 {
+    const Inside in;
     note(st, "copy " + std::to_string(n) + " to " + std::to_string(block_of(d)) + " from " + std::to_string(block_of(s)));
     std::memcpy(d, s, n);
     return hipSuccess;

@@ -40,6 +40,24 @@ for i, call in enumerate(calls):
 """ % (N, ROOM))
 
 
+@pytest.mark.skipif(not os.path.exists(host_hip.LIB), reason="libspns.so not built")
+@pytest.mark.parametrize("started", [0, 1, 2])
+def test_read_without_memory_for_its_threads(tmp_path, started):
+    # a thread that cannot be started is done without
+    host_hip.run(tmp_path, """
+s = spns_amd.Solver(Nx=96, Ny=64, Nz=64, nu=1e-3)
+s.get_state()
+out = np.empty((3, s.nmodes), complex)
+p = out.ctypes.data_as(ctypes.POINTER(ctypes.c_double))
+log()
+hip.host_hip_fail_alloc(%d)
+rc = s.L.spns_get_state(s.h, p)
+hip.host_hip_fail_alloc(-1)
+assert rc == 0, (rc, s.L.spns_last_error(s.h))
+assert len(kernels(log())) == -(-out.nbytes // (2 << 20))
+""" % started)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("prec", [0, 1])
 @pytest.mark.parametrize("N", [(32, 32, 32), (96, 64, 64)])
