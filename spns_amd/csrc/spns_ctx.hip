@@ -249,7 +249,21 @@ struct spns_fft {
     int Mx, My, Mz, prec, device;
     void *twx = nullptr, *twy = nullptr, *twz = nullptr;
     hipStream_t st = nullptr;
+    int grid_x[2], grid_y[2], grid_z[2];  // of the three passes, [dir > 0]
     std::string err;
+
+    // with the plan's device current
+    void init_grids()
+    {
+        const int64_t nk = Mz / 2 + 1;
+        for (int d = 0; d < 2; d++) {
+            const int dir = d ? +1 : -1;
+            grid_x[d] = line_grid(Mx, prec, dir, My, nk);
+            grid_y[d] = line_grid(My, prec, dir, 1, Mx * nk);
+            grid_z[d] = zline_grid(Mz, prec, dir, (int64_t)Mx * My);
+            if (grid_x[d] < 1 || grid_y[d] < 1 || grid_z[d] < 1) throw Error(SPNS_EHIP, "transform: no launch configuration");
+        }
+    }
 
     void fft_x(void* c, int dir)
     {
@@ -264,7 +278,7 @@ struct spns_fft {
         int64_t cap = (int64_t)My * Mx * nk;
         check_strided(a, My, &cap, &cap, 0);
         a.A = My;
-        HIPCHK(launch_line(Mx, prec, dir, a, st));
+        HIPCHK(launch_line(Mx, prec, dir, a, grid_x[dir > 0], st));
     }
     void fft_y(void* c, int dir)
     {
@@ -278,12 +292,12 @@ struct spns_fft {
         int64_t cap = (int64_t)My * Mx * nk;
         check_strided(a, 1, &cap, &cap, 0);
         a.A = 1;
-        HIPCHK(launch_line(My, prec, dir, a, st));
+        HIPCHK(launch_line(My, prec, dir, a, grid_y[dir > 0], st));
     }
     void z(const void* in, void* out, int dir)
     {
         const ZPlainArgs a{in, out, Mx, My, twz};
-        HIPCHK(launch_zplain(Mz, prec, dir, a, st));
+        HIPCHK(launch_zplain(Mz, prec, dir, a, grid_z[dir > 0], st));
     }
 };
 
@@ -1986,6 +2000,7 @@ int spns_fft_create(int32_t Mx, int32_t My, int32_t Mz, int32_t precision, int32
         f->twx = upload_twiddles(Mx, f->prec);
         f->twy = upload_twiddles(My, f->prec);
         f->twz = upload_twiddles(Mz, f->prec);
+        f->init_grids();
     } catch (const Error& e) {
         g_create_error = e.what();
         spns_fft_destroy(f);

@@ -193,8 +193,10 @@ hipError_t launch_zreg(int L, int prec, const ZArgs& a, int grid, hipStream_t st
 int zreg_blocks(int L, int prec, bool les);                                                                 // its blocks per CU
 int zpass_grid(int L, int prec, const ZArgs& a, int64_t npen);  // < 0: no such length / HIP error
 int zpass_kernel(int L, int prec, const ZArgs& a);              // kernel launch_zpass picks
-hipError_t launch_zplain(int L, int prec, int dir, const ZPlainArgs& a, hipStream_t st);
-hipError_t launch_line(int L, int prec, int dir, const StridedArgs& a, hipStream_t st);  // in place, unpruned, any row alignment
+int zline_grid(int L, int prec, int dir, int64_t np);             // of launch_zplain, np pencils; < 1: no such length / HIP error
+int line_grid(int L, int prec, int dir, int64_t A, int64_t B);    // of launch_line
+hipError_t launch_zplain(int L, int prec, int dir, const ZPlainArgs& a, int grid, hipStream_t st);
+hipError_t launch_line(int L, int prec, int dir, const StridedArgs& a, int grid, hipStream_t st);  // in place, unpruned, any row alignment
 // inv: the variant with the next step's inverse y pass (k_yepi_inv), which
 // launch_yepi runs when ia (the inverse pass's arguments) is given; it sets
 // *x1v

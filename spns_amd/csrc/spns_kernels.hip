@@ -3427,55 +3427,83 @@ static int resident_grid(Kern kern, int nt, int64_t items)
     return (int)((g + 7) / 8 * 8);
 }
 
+// The launches' grids, which ask the runtime for the device and the occupancy:
+// host time that a plan pays once (spns_fft keeps them).
 template <typename T, int L, int DIR>
-static hipError_t launch_zline_L(const ZPlainArgs& a, hipStream_t st)
+static int zline_grid_L(int64_t np)
 {
     constexpr int NB = zline_nb<T, L>(), NT = sstage_nt<L, NB>();
-    const int64_t np = (int64_t)a.Mx * a.My;
-    if (np >= ((int64_t)1 << 30)) return hipErrorInvalidValue;  // 32-bit pencil index
-    const int g = resident_grid(k_zline<T, L, NB, NT, DIR>, NT, ((np + 1) / 2 + NB - 1) / NB);
-    if (g < 1) return hipErrorUnknown;
-    hipLaunchKernelGGL((k_zline<T, L, NB, NT, DIR>), dim3(g), dim3(NT), 0, st, a);
+    if (np >= ((int64_t)1 << 30)) return -1;  // 32-bit pencil index
+    return resident_grid(k_zline<T, L, NB, NT, DIR>, NT, ((np + 1) / 2 + NB - 1) / NB);
+}
+
+template <typename T, int L, int DIR>
+static int line_grid_L(int64_t A, int64_t B)
+{
+    constexpr int TB = line_tb<T, L>(), NT = sstage_nt<L, TB>();
+    return resident_grid(k_line<T, L, TB, NT, DIR>, NT, A * ((B + TB - 1) / TB));
+}
+
+template <typename T, int L, int DIR>
+static hipError_t launch_zline_L(const ZPlainArgs& a, int grid, hipStream_t st)
+{
+    constexpr int NB = zline_nb<T, L>(), NT = sstage_nt<L, NB>();
+    if (grid < 1 || (int64_t)a.Mx * a.My >= ((int64_t)1 << 30)) return hipErrorInvalidValue;
+    hipLaunchKernelGGL((k_zline<T, L, NB, NT, DIR>), dim3(grid), dim3(NT), 0, st, a);
     return hipGetLastError();
 }
 
-hipError_t launch_zplain(int L, int prec, int dir, const ZPlainArgs& a, hipStream_t st)
-{
-#define X(LL)                                                                                        \
-    if (L == LL) {                                                                                   \
-        if (prec == PREC_FP64) return dir > 0 ? launch_zline_L<double, LL, +1>(a, st)                \
-                                              : launch_zline_L<double, LL, -1>(a, st);               \
-        return dir > 0 ? launch_zline_L<float, LL, +1>(a, st) : launch_zline_L<float, LL, -1>(a, st); \
-    }
-    SPNS_FOR_EACH_L(X)
-#undef X
-    return hipErrorInvalidValue;
-}
-
 template <typename T, int L, int DIR>
-static hipError_t launch_line_L(const StridedArgs& a, hipStream_t st)
+static hipError_t launch_line_L(const StridedArgs& a, int grid, hipStream_t st)
 {
     constexpr int TB = line_tb<T, L>(), NT = sstage_nt<L, TB>();
     static_assert(sizeof(cx<T>) * ((size_t)L * TB + L) <= 160 * 1024 - 512, "tile and table fit the LDS");
     if (a.njobs != 1 || a.nin != L || a.nout != L || a.job[0].out2 || a.job[0].deriv || a.job[0].in != a.job[0].out) return hipErrorInvalidValue;
-    const int g = resident_grid(k_line<T, L, TB, NT, DIR>, NT, (int64_t)a.A * ((a.B + TB - 1) / TB));
-    if (g < 1) return hipErrorUnknown;
-    hipLaunchKernelGGL((k_line<T, L, TB, NT, DIR>), dim3(g), dim3(NT), 0, st, a);
+    if (grid < 8 || grid % 8) return hipErrorInvalidValue;
+    hipLaunchKernelGGL((k_line<T, L, TB, NT, DIR>), dim3(grid), dim3(NT), 0, st, a);
     return hipGetLastError();
 }
 
-hipError_t launch_line(int L, int prec, int dir, const StridedArgs& a, hipStream_t st)
+#define X(LL)                                                                                              \
+    case LL:                                                                                               \
+        if (prec == PREC_FP64) return dir > 0 ? zline_grid_L<double, LL, +1>(np) : zline_grid_L<double, LL, -1>(np); \
+        return dir > 0 ? zline_grid_L<float, LL, +1>(np) : zline_grid_L<float, LL, -1>(np);
+int zline_grid(int L, int prec, int dir, int64_t np)
 {
-#define X(LL)                                                                                        \
-    if (L == LL) {                                                                                   \
-        if (prec == PREC_FP64) return dir > 0 ? launch_line_L<double, LL, +1>(a, st)                 \
-                                              : launch_line_L<double, LL, -1>(a, st);                \
-        return dir > 0 ? launch_line_L<float, LL, +1>(a, st) : launch_line_L<float, LL, -1>(a, st);  \
-    }
-    SPNS_FOR_EACH_L(X)
+    switch (L) { SPNS_FOR_EACH_L(X) }
+    return -1;
+}
 #undef X
+#define X(LL)                                                                                              \
+    case LL:                                                                                               \
+        if (prec == PREC_FP64) return dir > 0 ? line_grid_L<double, LL, +1>(A, B) : line_grid_L<double, LL, -1>(A, B); \
+        return dir > 0 ? line_grid_L<float, LL, +1>(A, B) : line_grid_L<float, LL, -1>(A, B);
+int line_grid(int L, int prec, int dir, int64_t A, int64_t B)
+{
+    switch (L) { SPNS_FOR_EACH_L(X) }
+    return -1;
+}
+#undef X
+#define X(LL)                                                                                              \
+    case LL:                                                                                               \
+        if (prec == PREC_FP64) return dir > 0 ? launch_zline_L<double, LL, +1>(a, grid, st) : launch_zline_L<double, LL, -1>(a, grid, st); \
+        return dir > 0 ? launch_zline_L<float, LL, +1>(a, grid, st) : launch_zline_L<float, LL, -1>(a, grid, st);
+hipError_t launch_zplain(int L, int prec, int dir, const ZPlainArgs& a, int grid, hipStream_t st)
+{
+    switch (L) { SPNS_FOR_EACH_L(X) }
     return hipErrorInvalidValue;
 }
+#undef X
+#define X(LL)                                                                                              \
+    case LL:                                                                                               \
+        if (prec == PREC_FP64) return dir > 0 ? launch_line_L<double, LL, +1>(a, grid, st) : launch_line_L<double, LL, -1>(a, grid, st); \
+        return dir > 0 ? launch_line_L<float, LL, +1>(a, grid, st) : launch_line_L<float, LL, -1>(a, grid, st);
+hipError_t launch_line(int L, int prec, int dir, const StridedArgs& a, int grid, hipStream_t st)
+{
+    switch (L) { SPNS_FOR_EACH_L(X) }
+    return hipErrorInvalidValue;
+}
+#undef X
 
 #endif
 
