@@ -1305,12 +1305,16 @@ __device__ __forceinline__ void z_pair_dz(cx<T> A, int k, cx<T>& lo, cx<T>& hi)
 
 // Pencils per block: two at the short DNS lengths, so that butterflies fill whole
 // waves (96^3 points, FP32: a run 84 us a step against 87 with one, 16 of them 654
-// against 670; four: 89 and 720), but one in FP64 at 96 and 144, where two hold
-// 126 VGPRs (16 x 64^3: 1.23 ms a step against 1.47, 64^3 alone 116 us against 125).
+// against 670; four: 89 and 720), but one in FP64 where two hold too many registers:
+// 126 VGPRs at 96 and 144 (16 x 64^3: 1.23 ms a step against 1.47, 64^3 alone 116 us
+// against 125), and 33 spilt at 36 (z pass of 96x96x24 33.7 us against 37.7, 24^3
+// 11.1 against 11.4).
 template <typename T, int L, bool LES>
 __host__ __device__ constexpr int zreg_pp()
 {
-    return LES ? 1 : L <= (sizeof(T) == 4 ? 144 : 72) ? 2 : 1;
+    if (LES) return 1;
+    if (sizeof(T) == 8) return L <= 72 && L != 36 ? 2 : 1;
+    return L <= 144 ? 2 : 1;
 }
 
 // Threads: one butterfly each in every stage after the first (whose radix is
