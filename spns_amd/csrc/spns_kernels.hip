@@ -1276,6 +1276,9 @@ __global__ __launch_bounds__(NT) void k_zfuse_b(const ZArgs* __restrict__ arr, c
 // short lengths (so PP is taken to fill whole waves with butterflies).
 // z pass, one run: 256^3 LES 2.93 -> 2.34 ms FP64, 1.43 -> 1.18 FP32; 192^3 DNS
 // FP64 1.01 -> 0.66; 128^3 DNS FP64 243 -> 181 us; 16 x 64^3 DNS FP32 359 -> 261 us.
+// Long LES pencils (192 x 192 of them; from 768 on 1024 threads spill in FP64, 20 to
+// 177 registers): 768 FP64 1.40 -> 1.27 ms, FP32 0.73 -> 0.65; 1152 9.5 -> 3.0, 1.38 ->
+// 1.11; 1536 13.7 -> 4.8, 1.78 -> 1.45 (FP64 there against the unstaged k_zpass).
 // ---------------------------------------------------------------------------
 // Pair (A, B) at k3 = k: Z[k] (lo) and Z[L - k] (hi) of A + i B; dza / dzb: the
 // field is d_z of the one read.  Only the real part of k3 = 0 enters (as in a
@@ -1784,7 +1787,8 @@ __global__ __launch_bounds__(256) void k_zwave(ZArgs a)
 // in a loop cost more than either: 4.1 ms for the r2c.
 // ---------------------------------------------------------------------------
 // Pairs per block: 8 at most, fewer where the exchange buffer would leave room
-// for less than three blocks per CU.
+// for less than three blocks per CU (two are the least: FP64 at 1152 and 1536 has
+// two blocks and one).
 template <typename T, int L>
 __host__ __device__ constexpr int zline_nb()
 {
@@ -2338,8 +2342,9 @@ struct YComb {
     static constexpr size_t bytes(int tb) { return sizeof(cx<T>) * L * (size_t)(NF > 6 ? NF : 6) * tb; }
     // 4 columns at the shortest lengths: 147 against 170 us a step for 16 x 32^3
     static constexpr int TB = L <= 48 || bytes(8) > 112 * 1024 ? 4 : 8;
-    // one butterfly a thread in every stage, as in the separate kernels: with two
-    // the compiler contracts some differently, and FP32 would not keep its bits
+    // one butterfly a thread in every stage as far as 1024 threads go (LES from 128
+    // on: two to five).  State and history are the separate kernels' bit for bit at
+    // every length; two a thread where one would do had changed FP32 bits.
     static constexpr int NT = sstage_nt<L, (NF > 6 ? NF : 6) * TB>();
     // state and history read before the forward transform: at the shortest
     // lengths (beyond, the registers cost more than the latency)
@@ -2349,7 +2354,11 @@ struct YComb {
     // DNS: from 96 points on the batched runs are faster with k_yepi's smaller
     // blocks (16 x 64^3 FP32: 691 against 838 us a step; one run 97 against 84).
     // LES, which has no other fused form: to 144 points, FP64 to 192 (128^3 870 ->
-    // 808 us; FP32 there 612 -> 606, but a batch of 16 7.80 -> 8.17 ms).
+    // 808 us; FP32 there 612 -> 606, but a batch of 16 7.80 -> 8.17 ms).  Several LES
+    // forms spill (1024 threads hold 128 VGPRs: 38 at 72 FP64, 19 at 128 FP32, up to
+    // 16 at 96, 144 and 192), and each is still faster than the separate kernels, a
+    // step: 48x48x64 at 72 FP64 89 against 104 us, 128x84x64 at 128 FP32 215 against
+    // 263, 8 x 96^3 at 144 FP32 1.55 against 1.77 ms, 8 x 128^3 FP64 6.10 against 6.53.
     static constexpr bool use = L <= (!LES ? 72 : sizeof(T) == 8 ? 192 : 144) && lds <= 144 * 1024;
 };
 
