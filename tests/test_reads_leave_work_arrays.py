@@ -41,6 +41,21 @@ for i, call in enumerate(calls):
 
 
 @pytest.mark.skipif(not os.path.exists(host_hip.LIB), reason="libspns.so not built")
+def test_fetch_is_one_copy(tmp_path):
+    # a batch's room holds a whole state of its class (26 MB here)
+    host_hip.run(tmp_path, """
+s = spns_amd.Solver(Nx=128, Ny=128, Nz=64, nu=1e-3)
+b = spns_amd.Batch(1, 2)
+b.attach(0, s)
+state = np.zeros((3, s.nmodes), complex)
+log()
+b.fetch(0, state)
+copies = [l.split() for l in log() if l.startswith("copy")]
+assert [int(c[1]) for c in copies] == [state.nbytes], copies
+""")
+
+
+@pytest.mark.skipif(not os.path.exists(host_hip.LIB), reason="libspns.so not built")
 @pytest.mark.parametrize("started", [0, 1, 2])
 def test_read_without_memory_for_its_threads(tmp_path, started):
     # a thread that cannot be started is done without
