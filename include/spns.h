@@ -3,7 +3,9 @@
  *
  * Plain pointers and sizes only.  Every call returns 0 on success or a
  * SPNS_E* code; spns_last_error() gives the message.  Calls on one context
- * are ordered on that context's HIP stream; use one host thread per context.
+ * are ordered on that context's HIP stream; use one host thread per context
+ * (calls of several threads on one context take turns).  A call runs on the
+ * context's device whichever device is current, and leaves that as it was.
  *
  * The reference (adalbal/SpNS) has no FFI: its seam is the C++ class surface
  * `main` uses.  Each entry point below names the reference member it replaces.
@@ -59,8 +61,8 @@ typedef struct spns_config {
     int32_t force_kmin, force_kmax;
     int32_t device;          /* HIP device ordinal */
     int32_t use_graph;       /* capture the step as a hipGraph */
-    int32_t zpass_variant;   /* z-pass kernel: 0 default (staged inputs; DNS forward folded into the next
-                                pencil's inverse), 1 block per pencil, 2 wave per pencil, 3 staged, not folded */
+    int32_t zpass_variant;   /* z-pass kernel: 0 default (inputs held in registers or staged; DNS forward folded
+                                into the next pencil's inverse), 1 block per pencil, 2 wave per pencil, 3 staged, not folded */
     int32_t gradient_invariants; /* keep the state at the start of each step (one more state copy per step)
                                     so spns_invariant_spectra can evaluate it */
     int32_t keep_step_start; /* keep it as well (implied by the two flags above) so that

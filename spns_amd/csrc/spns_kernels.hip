@@ -336,14 +336,14 @@ __global__ __launch_bounds__(NT) void k_sstage(StridedArgs a)
 // 58 -> 47 us, 48^3 26.0 -> 21.6 us.
 // ---------------------------------------------------------------------------
 // Columns per tile: 128-byte row pieces as far as the threads (at most 1024) and
-// the LDS go.  FP32: 16 to L = 512 (there 668 us a 512^3 transform against 811
+// the LDS go, which is L = 512.  FP32: 16 (there 668 us a 512^3 transform against 811
 // with 8), FP64: 8 (192^3: 76 us against 121 with 16, whose blocks have 1024
-// threads); beyond, the strided passes' tile.
+// threads; 512^3 r2c 1340 us against 1587 with 4, 256x512x256 392 against 484, where
+// the passes before these took 1547 and 455); beyond, the strided passes' tile.
 template <typename T, int L>
 __host__ __device__ constexpr int line_tb()
 {
-    constexpr int tb = strided_tb<T, L>();
-    return sizeof(T) == 4 ? (L <= 512 ? 16 : tb) : (tb < 8 ? tb : 8);
+    return L > 512 ? strided_tb<T, L>() : sizeof(T) == 4 ? 16 : 8;
 }
 
 template <typename T, int L, int TB, int NT, int DIR>
