@@ -1383,12 +1383,12 @@ struct OnDevice {
     try { \
         const std::lock_guard<std::mutex> one_call((c)->mu); \
         const OnDevice on_device((c)->cfg.device);
-// for calls that use no memory of the context but its scalars and spectrum: they
-// do not wait for another thread's call
+// for calls that launch nothing and use no memory of the context but its scalars
+// and spectrum: they do not wait for another thread's call, and copies and waits
+// on a stream need no current device
 #define API_OPEN(c) \
     if (!(c)) return SPNS_EINVAL; \
-    try { \
-        const OnDevice on_device((c)->cfg.device);
+    try {
 #define API_END(c)                                   \
     }                                                \
     catch (const Error& e) { return finish(c, e, e.code); } \
