@@ -1772,12 +1772,14 @@ static void physical_out(spns_ctx* ctx, double* uvw, bool step_start)
     char* room[2] = {(char*)ctx->X2f(3), (char*)ctx->X1};
     size_t left[2] = {(size_t)6 * ctx->x2_slot * ctx->tsz, (size_t)ctx->n_x1 * ctx->x1_slot * ctx->tsz};
     double* d[3] = {};
+    int in[3] = {-1, -1, -1};  // the room it lies in
     void* own[3] = {};
     try {
         for (int c = 0; c < 3; c++) {
             for (int r = 0; r < 2 && !d[c]; r++)
                 if (left[r] >= pb) {
                     d[c] = (double*)room[r];
+                    in[c] = r;
                     room[r] += pb;
                     left[r] -= pb;
                 }
@@ -1788,7 +1790,10 @@ static void physical_out(spns_ctx* ctx, double* uvw, bool step_start)
         }
         if (step_start) ctx->velocity_step_start(d);
         else ctx->velocity_pass(d);
-        for (int c = 0; c < 3; c++) ctx->hcopy.copy(uvw + c * P, pb, ctx->cfg.device, ctx->st, PlainPiece<true>{(char*)d[c]});
+        for (int c = 0, n; c < 3; c += n) {  // neighbours in one copy
+            for (n = 1; c + n < 3 && in[c] >= 0 && in[c + n] == in[c];) n++;
+            ctx->hcopy.copy(uvw + c * P, n * pb, ctx->cfg.device, ctx->st, PlainPiece<true>{(char*)d[c]});
+        }
     } catch (...) {
         hipStreamSynchronize(ctx->st);
         for (void* p : own) hipFree(p);

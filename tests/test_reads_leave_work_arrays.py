@@ -73,6 +73,18 @@ assert len(kernels(log())) == -(-out.nbytes // (2 << 20))
 """ % started)
 
 
+@pytest.mark.skipif(not os.path.exists(host_hip.LIB), reason="libspns.so not built")
+@pytest.mark.parametrize("prec", [0, 1])
+def test_small_velocity_is_one_copy(tmp_path, prec):
+    host_hip.run(tmp_path, """
+s = spns_amd.Solver(Nx=16, nu=1e-3, precision=%d)
+log()
+out = s.velocity_physical()
+copies = [l.split() for l in log() if l.startswith("copy")]
+assert [int(c[1]) for c in copies] == [out.nbytes], copies
+""" % prec)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("prec", [0, 1])
 @pytest.mark.parametrize("N", [(32, 32, 32), (96, 64, 64)])
