@@ -394,6 +394,8 @@ struct spns_ctx {
     // on the device)
     hipGraphExec_t graph[2] = {};
     bool x1_cur = false;
+    bool x1_set = false;   // a step since the last clear may have set x1v
+    bool batched = false;  // a batch may have, at any time since the context joined one
     HostCopy hcopy;
     char* room = nullptr;  // of small packed copies: a read of the state uses none of the passes' arrays
     std::mutex mu;         // held by every call that uses the passes' arrays, hcopy or room
@@ -636,7 +638,9 @@ struct spns_ctx {
     void x1_stale()
     {
         x1_cur = false;
-        if (yinv) HIPCHK(launch_set_int(x1v, 0, st));
+        if (!yinv || !(x1_set || batched)) return;
+        HIPCHK(launch_set_int(x1v, 0, st));
+        x1_set = false;
     }
 
     // x passes: rows = x (or i1), batch = (y outer, i3 contiguous)
@@ -793,6 +797,7 @@ struct spns_ctx {
     {
         if (yinv) {
             const StridedArgs ia = inv_y_args(false);
+            x1_set = true;
             HIPCHK(launch_yepi(My, prec, fwd_y_args(nfwd), nk1, epi_args(EPI_STEP), grid_yinv, st, nullptr, &ia, x1v));
             return grid_yinv;
         }
@@ -933,6 +938,7 @@ struct spns_ctx {
                     hipGraphDestroy(g);
                     HIPCHK(e);
                 }
+                x1_set = yinv;
                 HIPCHK(hipGraphLaunch(ge, st));
             } else {
                 enqueue_step(x1);
@@ -1161,6 +1167,7 @@ struct spns_batch {
         HIPCHK(hipStreamSynchronize(st));        // no copy in flight reads this slot's pinned structs
         c->x1_stale();                           // the first batched step runs the inverse y pass
         HIPCHK(hipStreamSynchronize(c->st));     // the context's own work is done
+        c->batched = true;
         if (!r) make_room(c->pack_bytes((int64_t)c->nk2 * c->nk1));
         SlotArgs& a = hs[s];
         a.invy = c->inv_y_args(false);
