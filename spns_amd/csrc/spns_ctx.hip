@@ -103,16 +103,17 @@ void check_strided(StridedArgs& a, int A, const int64_t* in_cap, const int64_t* 
 // 57 GB/s, but one hipMemcpy into freshly allocated pages 10.3 (512 MiB), where
 // the page faults and the host's own copy are serial; this moves 32 (52 and
 // 170 MB; six or eight threads the same).  Small ones are one hipMemcpy: below
-// kSmall the threads cost more than they save.
+// kSmallOut and kSmallIn the threads cost more than they save (6.7 MB out 367 us
+// against 479 with one hipMemcpy, in 325 against 261).
 // A Piece is the device side: move queues the copy of its bytes [off, off + n) from
 // or to pinned memory on st, move_by that from or to any host memory, by way of
-// device memory of its owner (room, kSmall bytes) where it has to.
+// device memory of its owner (room, kSmallOut bytes) where it has to.
 // The pinned memory (16 MiB) belongs to the owner and goes with it.
 // ===========================================================================
 namespace {
 struct HostCopy {
     static constexpr int kThreads = 4;
-    static constexpr size_t kChunk = 2u << 20, kSmall = 8u << 20;
+    static constexpr size_t kChunk = 2u << 20, kSmallOut = 4u << 20, kSmallIn = 8u << 20;
     char* pin = nullptr;  // [kThreads][2][kChunk]
     hipEvent_t ev[kThreads][2] = {};
 
@@ -121,6 +122,7 @@ struct HostCopy {
     void copy(void* host, size_t bytes, int device, hipStream_t st, const Piece& piece, char* room = nullptr)
     {
         constexpr bool to_host = Piece::to_host;
+        constexpr size_t kSmall = to_host ? kSmallOut : kSmallIn;
         if (bytes < kSmall || !ready()) {
             for (size_t off = 0; off < bytes; off += kSmall) {
                 const size_t n = std::min(kSmall, bytes - off);
@@ -497,7 +499,7 @@ struct spns_ctx {
         alloc((void**)&x1v, sizeof(int));
         alloc((void**)&ek, sizeof(double) * nbins);
         alloc((void**)&ft, sizeof(double) * (nbins + 1));
-        alloc((void**)&room, std::min(HostCopy::kSmall, pack_bytes((int64_t)nk2 * nk1)));
+        alloc((void**)&room, std::min(HostCopy::kSmallOut, pack_bytes((int64_t)nk2 * nk1)));
         HIPCHK(hipMemsetAsync(z_partial, 0, sizeof(double) * 4 * grid_z, st));
         HIPCHK(hipMemsetAsync(X1, 0, (size_t)n_x1 * x1_slot * tsz, st));
         HIPCHK(hipMemsetAsync(X2, 0, (size_t)9 * x2_slot * tsz, st));

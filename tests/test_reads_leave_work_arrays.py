@@ -75,6 +75,24 @@ assert len(kernels(log())) == -(-out.nbytes // (2 << 20))
 
 @pytest.mark.skipif(not os.path.exists(host_hip.LIB), reason="libspns.so not built")
 @pytest.mark.parametrize("prec", [0, 1])
+def test_threads_take_part_by_size(tmp_path, prec):
+    # outwards from 4 MiB, inwards from 8 MiB on: chunks of 2 MiB, else one copy
+    host_hip.run(tmp_path, """
+s = spns_amd.Solver(Nx=64, nu=1e-3, precision=%d)  # 6.7 MB
+state = np.zeros((3, s.nmodes), complex)
+log()
+s.get_state()
+assert kernels(log()).count("k_pack") == 4
+s.set_state(state)
+copies = [int(l.split()[1]) for l in log() if l.startswith("copy")]
+assert copies[0] == state.nbytes, copies
+s.get_state_planes(0, 30)  # 3.1 MB
+assert kernels(log()).count("k_pack") == 1
+""" % prec)
+
+
+@pytest.mark.skipif(not os.path.exists(host_hip.LIB), reason="libspns.so not built")
+@pytest.mark.parametrize("prec", [0, 1])
 def test_small_velocity_is_one_copy(tmp_path, prec):
     host_hip.run(tmp_path, """
 s = spns_amd.Solver(Nx=16, nu=1e-3, precision=%d)
