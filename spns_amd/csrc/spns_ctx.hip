@@ -3,6 +3,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <array>
 #include <cmath>
 #include <complex>
 #include <cstdio>
@@ -1145,15 +1146,16 @@ struct spns_batch {
         if (st) hipStreamDestroy(st);
     }
 
-    // a context joins the class if its shapes, model and kernel choices match
-    // the representative's
-    static bool same_class(const spns_ctx* a, const spns_ctx* b)
+    // What the chunk's launches depend on: shapes, model and kernel choices
+    using Class = std::array<int, 17>;
+    static Class class_of(const spns_ctx* c)
     {
-        return a->Nx == b->Nx && a->Ny == b->Ny && a->Nz == b->Nz && a->Mx == b->Mx && a->My == b->My && a->Mz == b->Mz &&
-               a->prec == b->prec && a->les == b->les && a->nfwd == b->nfwd && a->zkernel == b->zkernel &&
-               a->grid_z == b->grid_z && a->grid_epi == b->grid_epi && a->grid_yepi == b->grid_yepi && a->nbins == b->nbins &&
-               a->yinv == b->yinv && a->grid_yinv == b->grid_yinv && a->cfg.device == b->cfg.device;
+        return {c->Nx, c->Ny, c->Nz, c->Mx, c->My, c->Mz, c->prec, c->les, c->nfwd, c->zkernel, c->grid_z, c->grid_epi, c->grid_yepi,
+                c->nbins, c->yinv, c->grid_yinv, c->cfg.device};
     }
+    // a context joins the class if it matches the representative
+    static bool same_class(const spns_ctx* a, const spns_ctx* b) { return class_of(a) == class_of(b); }
+    Class graph_class{};  // of the captured chunk
 
     void attach(int s, spns_ctx* c)
     {
@@ -1170,6 +1172,12 @@ struct spns_batch {
         c->x1_stale();                           // the first batched step runs the inverse y pass
         HIPCHK(hipStreamSynchronize(c->st));     // the context's own work is done
         c->batched = true;
+        if (graph && class_of(c) != graph_class) {
+            // the chunk's graph holds the kernels and grids of a class that has left
+            // (it is idle: the stream was waited for)
+            HIPCHK(hipGraphExecDestroy(graph));
+            graph = nullptr;
+        }
         if (!r) make_room(c->pack_bytes((int64_t)c->nk2 * c->nk1));
         SlotArgs& a = hs[s];
         a.invy = c->inv_y_args(false);
@@ -1229,11 +1237,7 @@ struct spns_batch {
         bool any = false;
         for (spns_ctx* o : slot) any = any || o;
         if (!any) {
-            // the next context may be of another class, and the chunk's graph holds
-            // this class's kernels and grids (it is idle: the stream was waited for)
-            rep = nullptr;
-            if (graph) HIPCHK(hipGraphExecDestroy(graph));
-            graph = nullptr;
+            rep = nullptr;  // the next context may be of another class
         } else if (rep == nullptr || std::find(slot.begin(), slot.end(), rep) == slot.end())
             for (spns_ctx* o : slot) if (o) { rep = o; break; }
     }
@@ -1296,7 +1300,7 @@ struct spns_batch {
         if (!graph) {
             // the chunk's launches read only the device arrays and counters,
             // so one capture serves every later set of slots of the class
-            // (detach drops it with the last slot)
+            // (attach drops it for a context of another)
             hipGraph_t g;
             HIPCHK(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
             try {
@@ -1311,6 +1315,7 @@ struct spns_batch {
             const hipError_t e = hipGraphInstantiate(&graph, g, nullptr, nullptr, 0);
             hipGraphDestroy(g);
             HIPCHK(e);
+            graph_class = class_of(rep);
         }
         HIPCHK(launch_set_left(d_left, n, nslots, st));
         HIPCHK(hipGraphLaunch(graph, st));

@@ -158,6 +158,7 @@ hipError_t hipStreamDestroy(hipStream_t s) { delete (Stream*)s; return hipSucces
 hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
 hipError_t hipStreamBeginCapture(hipStream_t s, hipStreamCaptureMode)
 {
+    count("hipStreamBeginCapture");
     of(s)->capture = new std::vector<std::string>;
     return hipSuccess;
 }

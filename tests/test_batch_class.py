@@ -42,6 +42,28 @@ assert got == want, (got, want)
 
 
 @needs_lib
+def test_refilled_with_its_class_it_keeps_the_chunk(tmp_path):
+    # a capture must not meet another thread's context creation: callers that keep
+    # the two apart do so for a batch's first chunk only
+    host_hip.run(tmp_path, """
+def slot(N, **kw):
+    return spns_amd.Solver(Nx=N, nu=1e-3, precision=1, **kw)
+
+def captures(b, s):
+    b.attach(1, s)
+    log()
+    b.step([0, 2])
+    n = log().count("call hipStreamBeginCapture")
+    b.detach(1)
+    return n
+
+b = spns_amd.Batch(2, 2)
+got = [captures(b, s) for s in (slot(32), slot(32), slot(32, omega=(0.0, 0.0, 1.0), force_eps=0.1), slot(64), slot(64), slot(32))]
+assert got == [1, 0, 0, 1, 0, 1], got
+""")
+
+
+@needs_lib
 def test_replaced_context_gives_the_class_no_more(tmp_path):
     host_hip.run(tmp_path, """
 a, b, c = [spns_amd.Solver(Nx=32, nu=1e-3, precision=1) for _ in range(3)]
