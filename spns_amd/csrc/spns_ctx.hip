@@ -103,7 +103,7 @@ void check_strided(StridedArgs& a, int A, const int64_t* in_cap, const int64_t* 
 // through pinned chunks that kThreads host threads fill or empty: the link moves
 // 57 GB/s, but one hipMemcpy into freshly allocated pages 10.3 (512 MiB), where
 // the page faults and the host's own copy are serial; this moves 32 (52 and
-// 170 MB; six or eight threads the same).  Small ones are one hipMemcpy: below
+// 170 MB; six or eight threads the same), 44 into pages that are there.  Small ones are one hipMemcpy: below
 // kSmallOut and kSmallIn the threads cost more than they save (6.7 MB out 367 us
 // against 479 with one hipMemcpy, in 325 against 261).
 // A Piece is the device side: move queues the copy of its bytes [off, off + n) from
